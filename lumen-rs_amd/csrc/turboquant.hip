@@ -644,82 +644,6 @@ __global__ void tq_values_kernel(const float* __restrict__ R, Codes code,
   out[i] = acc;
 }
 
-// The reference GPU cache's encode chain: lloyd_max_quantize_stage1
-// (turboquant.rs:398-423) over y = x (mode 0), over y = bf16(x M) (mode 1:
-// rotate_last_axis, then the encode) or over y = x M kept in f32 (mode 2:
-// rotate_and_lloyd_max_quantize_stage1_fused, :720-745), M = R or R^T
-// (transpose). sigma = sqrt(sum y^2 / D); code = the number of inner
-// boundaries b (ascending, f32) with b <= bf16(y / sigma) (the level scan of
-// lloyd_max_boundaries_inner, :310-331). One wavefront per kEncRows rows,
-// lane l holding channels l + 64 k of each (each load of M serves them
-// all): the rotation is tq_rotate_rows_kernel's fmaf chain over j from 0.0;
-// the sum of squares runs over k in each lane, then over the lanes by an
-// xor butterfly 32, 16, ..., 1 (MLX's own reduction order is not in the
-// reference; this one is fixed, and the oracle restates it).
-constexpr int kEncRows = 4;
-template <int D>
-__global__ __launch_bounds__(kWave) void tq_encode_gpu_kernel(
-    const uint16_t* __restrict__ x, int64_t s, int64_t rows, const float* __restrict__ R,
-    int mode, int transpose, const float* __restrict__ inner, int n_inner,
-    uint8_t* __restrict__ codes, float* __restrict__ sigma, int64_t dst_cap, int64_t dst_start) {
-  constexpr int PER = D / kWave;
-  __shared__ float xs[kEncRows][D];
-  __shared__ float bnd[256];
-  const int64_t r0 = int64_t(blockIdx.x) * kEncRows;
-  const int nr = rows - r0 < kEncRows ? int(rows - r0) : kEncRows;
-  const int lane = threadIdx.x;
-  for (int q = 0; q < kEncRows; ++q)
-    for (int i = lane; i < D; i += kWave)
-      xs[q][i] = q < nr ? bf16_to_f32(x[(r0 + q) * D + i]) : 0.0f;
-  for (int i = lane; i < n_inner; i += kWave) bnd[i] = inner[i];
-  __syncthreads();
-  float y[kEncRows][PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int i = lane + k * kWave;
-    if (mode == 0) {
-#pragma unroll
-      for (int q = 0; q < kEncRows; ++q) y[q][k] = xs[q][i];
-    } else {
-      float acc[kEncRows] = {};
-      for (int j = 0; j < D; ++j) {
-        const float rv = transpose ? R[int64_t(i) * D + j] : R[int64_t(j) * D + i];
-#pragma unroll
-        for (int q = 0; q < kEncRows; ++q) acc[q] = fmaf(xs[q][j], rv, acc[q]);
-      }
-#pragma unroll
-      for (int q = 0; q < kEncRows; ++q)
-        y[q][k] = mode == 1 ? bf16_to_f32(f32_to_bf16(acc[q])) : acc[q];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < kEncRows; ++q) {
-    if (q >= nr) break;
-    const int64_t r = r0 + q;
-    float p = 0.0f;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) p = add(p, mul(y[q][k], y[q][k]));
-#pragma unroll
-    for (int off = kWave / 2; off >= 1; off >>= 1) p = add(p, __shfl_xor(p, off, kWave));
-    const float sg = sqrt_rn(div_rn(p, float(D)));
-    const int64_t dst = (r / s) * dst_cap + dst_start + r % s;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const float xn = bf16_to_f32(f32_to_bf16(div_rn(y[q][k], sg)));
-      int lo = 0, hi = n_inner;
-      while (lo < hi) {
-        const int mid = (lo + hi) / 2;
-        if (bnd[mid] <= xn)
-          lo = mid + 1;
-        else
-          hi = mid;
-      }
-      codes[dst * D + lane + k * kWave] = uint8_t(lo);
-    }
-    if (lane == 0) sigma[dst] = sg;
-  }
-}
-
 // y = x R (x bf16 [rows, D] -> bf16): the GPU path's rotate_last_axis
 // (turboquant.rs:258-267), f32 accumulation. transpose = 1 applies R^T.
 __global__ void tq_rotate_rows_kernel(const uint16_t* __restrict__ x, int64_t rows, int D,
@@ -788,41 +712,6 @@ extern "C" int32_t tqkv_tq_encode(const void* x, int32_t x_is_bf16, int64_t n_sl
     hipLaunchKernelGGL(tq_encode_kernel<DIM>, dim3(unsigned(rows)), dim3(kWave), 0, st, x,   \
                        x_is_bf16, s, rotation, boundaries, centroids_f32, n, qjl, qjl_m,     \
                        codes, sigma, signs, rnorm, dst_cap, dst_start);                      \
-    break;
-  switch (dim) {
-    TQKV_ENC(64) TQKV_ENC(128) TQKV_ENC(256) TQKV_ENC(512)
-  }
-#undef TQKV_ENC
-  TQKV_LAUNCHED();
-  return ok();
-}
-
-extern "C" int32_t tqkv_tq_encode_gpu_path(const uint16_t* x, int64_t n_slabs, int64_t s,
-                                           int32_t dim, const float* rotation, int32_t mode,
-                                           int32_t transpose, const float* boundaries_inner,
-                                           int32_t bits, uint8_t* codes, float* sigma,
-                                           int64_t dst_cap, int64_t dst_start,
-                                           tqkv_stream stream) {
-  if (bits < 1 || bits > 8) return fail(TQKV_EUNSUPPORTED, "codebook bits=%d", bits);
-  if (!(dim == 64 || dim == 128 || dim == 256 || dim == 512))
-    return fail(TQKV_EUNSUPPORTED, "encode dim=%d not in {64,128,256,512}", dim);
-  if (mode < 0 || mode > 2) return fail(TQKV_EINVAL_ARG, "mode=%d not in {0, 1, 2}", mode);
-  if (n_slabs < 0 || s < 0 || dst_start < 0 || dst_start + s > dst_cap)
-    return fail(TQKV_EINVAL_SHAPE, "rows [%lld, %lld) do not fit a buffer of %lld",
-                (long long)dst_start, (long long)(dst_start + s), (long long)dst_cap);
-  if (n_slabs == 0 || s == 0) return ok();
-  if (!x || !boundaries_inner || !codes || !sigma || (mode != 0 && !rotation))
-    return fail(TQKV_EINVAL_ARG, "null pointer");
-  const int64_t rows = n_slabs * s;
-  if (rows > 0x7fffffffLL) return fail(TQKV_EINVAL_SHAPE, "too many rows");
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const int n_inner = (1 << bits) - 1;
-#define TQKV_ENC(DIM)                                                                       \
-  case DIM:                                                                                  \
-    hipLaunchKernelGGL(tq_encode_gpu_kernel<DIM>,                                            \
-                       dim3(unsigned((rows + kEncRows - 1) / kEncRows)), dim3(kWave), 0, st, x,  \
-                       s, rows, rotation, mode, transpose ? 1 : 0, boundaries_inner, n_inner,    \
-                       codes, sigma, dst_cap, dst_start);                                       \
     break;
   switch (dim) {
     TQKV_ENC(64) TQKV_ENC(128) TQKV_ENC(256) TQKV_ENC(512)

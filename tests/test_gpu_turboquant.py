@@ -290,6 +290,39 @@ def test_gpu_path_encode_bit_exact(T, mode, transpose, bits, D):
     assert np.all(gs[:, :start] == -7.0) and np.all(gs[:, start + s:] == -7.0)
 
 
+@pytest.mark.parametrize("D,rows,mode,transpose,off", [
+    (64, 17, 1, True, 0), (64, 8209, 1, False, 0), (128, 8192, 1, True, 0),
+    (128, 8193, 1, True, 0), (128, 8255, 2, False, 2), (256, 8200, 1, False, 0),
+    (512, 8193, 2, True, 0), (512, 15, 1, True, 2), (256, 33, 0, False, 2)])
+def test_gpu_path_encode_row_blocks(T, D, rows, mode, transpose, off):
+    # Both row-block sizes of the encode (16 rows, and 64 from 8,193 rows on
+    # at D > 64) and their remainders, on 16-byte aligned buffers and on ones
+    # `off` bytes past that (element-wise loads and byte stores): codes and
+    # sigma bit for bit, with a row of zeros (sigma 0, codes 0) and one whose
+    # values are subnormal in bf16.
+    bits = 4
+    print(f"[tq-gpu-path] rows={rows} D={D} mode={mode} transpose={transpose} off={off}", flush=True)
+    x = O.bf16_from_f32(np.random.default_rng(D + rows).standard_normal((rows, D)).astype(
+        np.float32))
+    x[3] = 0
+    x[5] &= 0x807F  # exponent 0: subnormals of both signs
+    R = T.rotation_matrix(D, 42)
+    inner = np.asarray(T.lloyd_max(bits)[0][1:-1]).astype(np.float32)
+    raw = np.zeros(rows * D + 8, np.uint16)
+    raw[off // 2:off // 2 + rows * D] = x.reshape(-1)
+    dx, dR, di = T.DeviceArray.of(raw), T.DeviceArray.of(R), T.DeviceArray.of(inner)
+    codes = T.DeviceArray((rows * D + 16,), np.uint8, np.full((rows * D + 16,), 0xAB, np.uint8))
+    sigma = T.DeviceArray((rows,), np.float32)
+    T.tq_encode_gpu_path(dx.ptr + off, 1, rows, D, dR.ptr, mode, transpose, di.ptr, bits,
+                         codes.ptr + off, sigma.ptr)
+    T.hip().sync()
+    wc, ws = O.tq_encode_gpu_path(x, inner, R, mode=mode, transpose=transpose)
+    gc = codes.numpy()
+    assert np.array_equal(gc[off:off + rows * D].reshape(rows, D), wc)
+    assert np.array_equal(sigma.numpy().view(np.uint32), ws.view(np.uint32))
+    assert np.all(gc[:off] == 0xAB) and np.all(gc[off + rows * D:] == 0xAB)
+
+
 def test_gpu_path_fused_matches_rotate_then_encode(T):
     # The reference's own test of its rotate+encode kernel
     # (turboquant.rs:1385-1456), on the device outputs: [1, 8, 64, 256] bf16
