@@ -29,7 +29,7 @@ KernelFn pick(int D, int bk, int bv, bool h16 = false) {
 // as bf16 rows [B * H_kv, slab_rows, D] with mlx::dequantize's arithmetic
 // (bf16(fma(scale, code, bias)), one rounding), V into vd as the prefill
 // kernel's V operands (those bf16 values times 2^-kVShift, in f16; see
-// v_operand_run): rows like K, or with vt (D = 128) transposed 64-key tiles
+// v_operand_run): rows like K, or with vt (D >= 128) transposed key tiles
 // (width kPreF16T; slab_rows a multiple of 64, zeros past the last key).
 // Grid: (row-run chunks, slab, K and/or V); a thread takes one run of 32
 // values of one row: its BITS words in one or two wide loads, its group's
@@ -49,20 +49,28 @@ __global__ __launch_bounds__(256) void dequantize_rows_kernel(const Args a, int 
   constexpr int kRuns = D / 32;
   static_assert(64 % kRuns == 0, "a wavefront covers whole rows");
   constexpr int kChunkRows = D / 8;  // 16-byte chunks a row
-  constexpr int KSTR = kKStride<D>;
-  // A wavefront's 64 runs x 4 chunks each (rows), or the tile's 64 keys
-  // row-major at the prefill kernel's stride (V^T).
-  constexpr int kLds = D == 128 ? 64 * KSTR / 8 : 1024;
+  // A V^T workgroup's channels and keys, and its row stride in LDS.
+  constexpr int kVtCh = D == 128 ? 128 : 256, kVtKeys = 8192 / kVtCh;
+  constexpr int KSTR = kKStride<kVtCh>;
+  // A wavefront's 64 runs x 4 chunks each (rows), or the workgroup's keys
+  // row-major (V^T).
+  constexpr int kLds = D >= 128 ? kVtKeys * KSTR / 8 : 1024;
   __shared__ uint4 s_buf[kLds];
   const int wv = threadIdx.x / 64, l = threadIdx.x % 64;
   const uint32_t j = blockIdx.x * 256u + threadIdx.x;
   const uint32_t total = uint32_t(a.total);
   if (total == 0) return;  // (uniform: no wavefront reaches the exchange)
-  const uint32_t row = j / kRuns;
-  const uint32_t lrow = row < total ? row : total - 1;  // past the end: load a live row
-  const int run = int(j % kRuns);
   const int slab = int(blockIdx.y), bb = slab / a.H_kv, kv = slab % a.H_kv;
   const bool isv = kinds == 3 ? blockIdx.z != 0 : kinds == 2;
+  uint32_t row = j / kRuns;
+  int run = int(j % kRuns);
+  constexpr int kVtRuns = kVtCh / 32;           // runs of a key a V^T workgroup takes
+  constexpr int kVtParts = D >= 128 ? D / kVtCh : 1;  // V^T workgroups a key block
+  if (D > kVtCh && isv && vt) {  // channel part blockIdx.x % kVtParts of its keys
+    row = blockIdx.x / kVtParts * kVtKeys + threadIdx.x / kVtRuns;
+    run = int(blockIdx.x % kVtParts) * kVtRuns + int(threadIdx.x % kVtRuns);
+  }
+  const uint32_t lrow = row < total ? row : total - 1;  // past the end: load a live row
   const bool first = lrow < uint32_t(a.n0);
   const Seg& s = a.seg[first ? 0 : 1];
   const int64_t src = int64_t(bb) * s.b_stride + int64_t(kv) * s.cap +
@@ -76,12 +84,12 @@ __global__ __launch_bounds__(256) void dequantize_rows_kernel(const Args a, int 
     v_operand_run<BITS>(w, sb, out);
   else
     dequant_run<BITS, false>(w, sb, out);
-  if constexpr (D == 128) {
+  if constexpr (D >= 128) {
     if (isv && vt) {  // (block-uniform)
       // Keys past the end are zeros: their weights are exactly 0, and 0
       // times a zero operand stays 0.
-      const int key = int(threadIdx.x) / kRuns;
-      uint4* d = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(s_buf) + key * KSTR + run * 32);
+      const int key = int(threadIdx.x) / kVtRuns, ch = int(threadIdx.x) % kVtRuns * 32;
+      uint4* d = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(s_buf) + key * KSTR + ch);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         d[i] = row < total ? uint4{out[4 * i], out[4 * i + 1], out[4 * i + 2], out[4 * i + 3]}
@@ -89,18 +97,22 @@ __global__ __launch_bounds__(256) void dequantize_rows_kernel(const Args a, int 
       __syncthreads();
       // Store pass (u, tt) of wavefront wv: lane (grp, lr) takes channel
       // 16 tt + lr of keys 32 u + 4 grp + [0, 4) and 32 u + 16 + 4 grp +
-      // [0, 4) (two transposing reads), the 16 bytes at slot 8 grp of V^T
-      // row u D + 16 tt + lr; the wavefront's 64 chunks are 16 whole rows.
+      // [0, 4) (two transposing reads), the 16 bytes at slot 8 grp of that
+      // channel's row in 32-key block u; the wavefront's 64 chunks are 16
+      // whole rows.
       const int grp = l / 16, lr = l % 16;
-      uint4* tile = reinterpret_cast<uint4*>(vd + (int64_t(slab) * slab_rows + int64_t(blockIdx.x) * kTile) * D);
+      const int c0 = int(blockIdx.x % kVtParts) * kVtCh;
+      uint4* tile = reinterpret_cast<uint4*>(
+          vd + (int64_t(slab) * slab_rows + int64_t(blockIdx.x / kVtParts) * kVtKeys) * D);
       const uint16_t* sv = reinterpret_cast<const uint16_t*>(s_buf);
+      constexpr int kTt = kVtCh / 16;
 #pragma unroll
       for (int it = 0; it < 4; ++it) {
-        const int pass = 4 * wv + it, u = pass / 8, tt = pass % 8;
+        const int pass = 4 * wv + it, u = pass / kTt, tt = pass % kTt;
         const uint16_t* vrow = sv + (32 * u + 4 * grp + lr / 4) * KSTR + 16 * tt + 4 * (lr % 4);
         const u32x2_t lo = tr_read(vrow);
         const u32x2_t hi = tr_read(vrow + 16 * KSTR);
-        tile[(u * D + 16 * tt + lr) * 4 + grp] = uint4{lo.x, lo.y, hi.x, hi.y};
+        tile[(u * D + c0 + 16 * tt + lr) * 4 + grp] = uint4{lo.x, lo.y, hi.x, hi.y};
       }
       return;
     }
@@ -141,22 +153,24 @@ void launch_dequantize_rows(const Args& a, int bits, int kinds, int64_t slab_row
 #undef TQKV_DQ
 }
 
-// V as transposed tiles (width kPreF16T) at this head dim.
-constexpr bool v_tiles(int D) { return D == 128; }
 // Rows a slab of the dequantize-once scratch holds: total, padded to whole
-// 64-key tiles where V is tiled (K shares the stride).
-int64_t once_slab_rows(int D, int64_t total) {
-  return v_tiles(D) ? (total + kTile - 1) / kTile * kTile : total;
+// 64-key tiles where V is tiled (width kPreF16T; K shares the stride).
+int64_t once_slab_rows(bool tiled, int64_t total) {
+  return tiled ? (total + kTile - 1) / kTile * kTile : total;
+}
+size_t once_bytes(int64_t slabs, int64_t slab_rows, int D) {
+  return 2 * size_t(slabs) * size_t(slab_rows) * size_t(D) * 2;
 }
 
 // Both halves of the dequantize-once pass: one launch when K and V share a
-// width, else one each. (At D = 128 a chunk of 256 runs is one 64-key tile.)
+// width, else one each.
 template <int D>
-void dequantize_rows(const Args& a, int bk, int bv, int64_t slabs, hipStream_t st, uint16_t* kd,
-                     uint16_t* vd) {
-  const unsigned chunks = unsigned((a.total * (D / 32) + 255) / 256);
-  const int64_t sr = once_slab_rows(D, a.total);
-  const int vt = v_tiles(D) ? 1 : 0;
+void dequantize_rows(const Args& a, int bk, int bv, int64_t slabs, bool tiled, hipStream_t st,
+                     uint16_t* kd, uint16_t* vd) {
+  const int64_t sr = once_slab_rows(tiled, a.total);
+  // (Tiled V: whole 64-key blocks, so that every tile is written.)
+  const unsigned chunks = unsigned((sr * (D / 32) + 255) / 256);
+  const int vt = tiled ? 1 : 0;
   if (bk == bv) {
     launch_dequantize_rows<D>(a, bk, 3, sr, vt, dim3(chunks, unsigned(slabs), 2), st, kd, vd);
   } else {
@@ -396,14 +410,21 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   // TQKV_PREFILL_DEQUANT_ONCE=0 / 1 forces the choice (tests compare them).
   const char* once_env = getenv("TQKV_PREFILL_DEQUANT_ONCE");
   const int64_t slabs = int64_t(B) * H_kv;
-  const int64_t slab_rows = once_slab_rows(D, a.total);
-  const size_t need = 2 * size_t(slabs) * size_t(slab_rows) * size_t(D) * 2;
+  // V as transposed tiles: always at D = 128; at D = 256 and 512 (the wide
+  // kernel) wherever the scratch has room for whole tiles, which the
+  // library's own has and a caller's workspace of
+  // tqkv_prefill_workspace_size bytes has for whole numbers of 64 keys.
+  const size_t tiled_bytes = once_bytes(slabs, once_slab_rows(true, a.total), D);
+  const bool tiled = D == 128 || (D > 128 && (library_scratch || workspace_bytes >= tiled_bytes));
+  const int64_t slab_rows = once_slab_rows(tiled, a.total);
+  const size_t need = once_bytes(slabs, slab_rows, D);
   // With a caller workspace (the _ws entry) the dequantized rows go there
   // when it holds them, else every block dequantizes for itself.
   const bool fits = library_scratch || (workspace && workspace_bytes >= need);
   const bool once = !bf16_rows && fits &&
                     (once_env ? strcmp(once_env, "0") != 0
-                              : blocks >= kOnceBlocks && need <= kOnceMaxBytes);
+                              : blocks >= kOnceBlocks &&
+                                    once_bytes(slabs, a.total, D) <= kOnceMaxBytes);
   if (once) {
     void* ws = workspace;
     if (library_scratch)
@@ -412,10 +433,10 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
     uint16_t* vd = kd + size_t(slabs) * size_t(slab_rows) * size_t(D);
     if (slabs > 65535) return fail(TQKV_EINVAL_SHAPE, "B * H_kv = %lld slabs", (long long)slabs);
     switch (D) {
-      case 64: dequantize_rows<64>(a, bits_k, bits_v, slabs, st, kd, vd); break;
-      case 128: dequantize_rows<128>(a, bits_k, bits_v, slabs, st, kd, vd); break;
-      case 256: dequantize_rows<256>(a, bits_k, bits_v, slabs, st, kd, vd); break;
-      default: dequantize_rows<512>(a, bits_k, bits_v, slabs, st, kd, vd); break;
+      case 64: dequantize_rows<64>(a, bits_k, bits_v, slabs, tiled, st, kd, vd); break;
+      case 128: dequantize_rows<128>(a, bits_k, bits_v, slabs, tiled, st, kd, vd); break;
+      case 256: dequantize_rows<256>(a, bits_k, bits_v, slabs, tiled, st, kd, vd); break;
+      default: dequantize_rows<512>(a, bits_k, bits_v, slabs, tiled, st, kd, vd); break;
     }
     TQKV_LAUNCHED();
     Args p = a;
@@ -425,8 +446,19 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
                    int64_t(H_kv) * slab_rows};
     p.seg[1] = p.seg[0];
     p.n0 = a.total;
-    hipLaunchKernelGGL(pick(D, kPreBits, v_tiles(D) ? kPreF16T : kPreF16), dim3(unsigned(grid)),
-                       dim3(threads), 0, st, p);
+    if (D >= 256 && tiled) {
+      // 64-row blocks where 128-row ones would not give every CU a workgroup
+      // (32 / 2 heads, D = 512, 512 rows over 8,192 keys: 380 us with 128
+      // rows, 331 with 64).
+      const int64_t q_rows = int64_t(L) * a.G;
+      const int wide_rows = (q_rows + 127) / 128 * H_kv * B >= 256 ? 128 : 64;
+      p.n_blocks = int((q_rows + wide_rows - 1) / wide_rows);
+      hipLaunchKernelGGL(pick_wide(D, wide_rows), dim3(unsigned(p.n_blocks * int64_t(H_kv) * B)),
+                         dim3(4 * wide_rows), 0, st, p);
+    } else {
+      hipLaunchKernelGGL(pick(D, kPreBits, tiled ? kPreF16T : kPreF16), dim3(unsigned(grid)),
+                         dim3(threads), 0, st, p);
+    }
     TQKV_LAUNCHED();
     return ok();
   }
@@ -451,7 +483,7 @@ extern "C" int32_t tqkv_prefill_attend_affine(const uint16_t* q, int32_t B, int3
 extern "C" size_t tqkv_prefill_workspace_size(int32_t B, int32_t H_kv, int32_t D,
                                               int64_t total_keys) {
   if (B <= 0 || H_kv <= 0 || D <= 0 || total_keys <= 0) return 0;
-  return 2 * size_t(B) * size_t(H_kv) * size_t(once_slab_rows(D, total_keys)) * size_t(D) * 2;
+  return once_bytes(int64_t(B) * H_kv, once_slab_rows(D == 128, total_keys), D);
 }
 
 extern "C" int32_t tqkv_prefill_attend_affine_ws(

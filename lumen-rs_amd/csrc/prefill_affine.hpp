@@ -257,7 +257,7 @@ struct Stage {
 // f16 values already in the prefill variant's V operand form (bf16 values
 // times 2^-kVShift, written once per (batch row, KV head) by
 // dequantize_rows_kernel), which the loaders copy into LDS as they are.
-// Width 18 (D = 128): the same V operands as transposed 64-key tiles, the
+// Width 18 (D >= 128): the same V operands as transposed 64-key tiles, the
 // slab padded to whole tiles (zeros past the last key). Tile t is 2 D rows
 // of 32 values: row u D + c holds channel c of keys 64 t + 32 u + [0, 32)
 // in the order of the P operand's k slots (slot 8 g + s: key 4 g + s for
@@ -1319,12 +1319,17 @@ void prefill_affine_kernel(const Args a) {
 typedef void (*KernelFn)(Args);
 
 // The kernel for (D, bits_k, bits_v), bits in {2, 3, 4, 5, 6, 8}, or
-// (kPreBits, kPreBits) / (kPreBits, kPreF16) for rows dequantized
-// beforehand; null if unsupported. h16: the f16-operand variant.
+// (kPreBits, kPreBits), (kPreBits, kPreF16) at D != 128 or (kPreBits,
+// kPreF16T) at D = 128 for rows dequantized beforehand (pick_wide above
+// takes kPreF16T at D = 256 and 512); null if unsupported. h16: the f16-operand variant.
 KernelFn pick_d64(int bk, int bv, bool h16);
 KernelFn pick_d128(int bk, int bv, bool h16);
 KernelFn pick_d256(int bk, int bv, bool h16);
 KernelFn pick_d512(int bk, int bv, bool h16);
+// The kernel of prefill_wide.hip for D = 256 or 512 (keys dequantized
+// beforehand, V as transposed tiles) at 64 or 128 rows a block, 4 threads a
+// row.
+KernelFn pick_wide(int D, int rows);
 
 template <int D, int BK, bool H16>
 KernelFn pick_bv(int bv) {
@@ -1343,7 +1348,8 @@ template <int D, bool H16>
 KernelFn pick_for(int bk, int bv) {
   if constexpr (!H16) {
     if (bk == kPreBits && bv == kPreBits) return prefill_affine_kernel<D, kPreBits, kPreBits, false>;
-    if (bk == kPreBits && bv == kPreF16) return prefill_affine_kernel<D, kPreBits, kPreF16, false>;
+    if constexpr (D != 128)
+      if (bk == kPreBits && bv == kPreF16) return prefill_affine_kernel<D, kPreBits, kPreF16, false>;
     if constexpr (D == 128)
       if (bk == kPreBits && bv == kPreF16T) return prefill_affine_kernel<D, kPreBits, kPreF16T, false>;
   }

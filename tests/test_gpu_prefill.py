@@ -208,6 +208,44 @@ def test_cache_prefill_rejects(T):
     assert e.value.status == T.EINVAL_SHAPE
 
 
+@pytest.mark.parametrize("B,H,Hkv,D,L,N,q_start,causal,window", [
+    (2, 32, 16, 256, 513, 1100, 587, True, -1),   # 128-row blocks, a 2-row last block
+    (2, 32, 16, 256, 520, 831, 311, True, 300),   # 128-row blocks, window
+    (1, 32, 8, 512, 1031, 1095, 64, True, -1),    # 128-row blocks, keys 7 past a tile
+    (1, 32, 8, 512, 1024, 1024, 0, False, -1),    # 128-row blocks, unmasked
+    (1, 8, 2, 256, 255, 63, 0, False, -1),        # 64-row blocks, fewer keys than a tile
+    (1, 16, 2, 512, 129, 191, 62, True, 65)])     # 64-row blocks, window across tiles
+def test_prefill_wide_heads_match_in_block(T, monkeypatch, B, H, Hkv, D, L, N, q_start, causal,
+                                           window):
+    # Head dims 256 and 512 over keys dequantized once (both row-block sizes,
+    # ragged last blocks and tiles) against the kernel that dequantizes in
+    # every block: the same products in the same order, so the same bits.
+    print(f"[prefill-wide] B={B} H={H}/{Hkv} D={D} L={L} N={N} window={window}", flush=True)
+    q = kv_bf16((B, H, L, D), D + L)
+    k = kv_bf16((B, Hkv, N, D), D + L + 1, frac=0.01, mult=10.0)
+    v = kv_bf16((B, Hkv, N, D), D + L + 2, frac=0.01, mult=10.0)
+    (kh, kd), (vh, vd) = _cache(k, 64, 4, N + 5), _cache(v, 64, 4, N + 5)
+    got = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("TQKV_PREFILL_DEQUANT_ONCE", mode)
+        got[mode] = run(T, q, [(kd, vd, N + 5, N, False)], B, H, Hkv, L, D, 64, 4, 4, D ** -0.5,
+                        q_start, 0, causal, window)
+    assert np.array_equal(got["0"], got["1"])
+    assert np.all(np.isfinite(O.bf16_to_f32(got["1"]))) and np.any(got["1"])
+    # A caller's workspace: exactly the stated bytes (whole tiles only at a
+    # multiple of 64 keys, else V as rows), and with room for whole tiles.
+    need = T.prefill_workspace_size(B, Hkv, D, N)
+    dq = T.DeviceArray.of(q)
+    seg = T.affine_seg(tuple(a.ptr for a in kd), tuple(a.ptr for a in vd), N + 5, N)
+    for ws_bytes in (need, 2 * B * Hkv * ((N + 63) // 64 * 64) * D * 2):
+        ws = T.DeviceArray((ws_bytes,), np.uint8)
+        out = T.DeviceArray((B, H, L, D), np.uint16, np.full((B, H, L, D), 0x7FC0, np.uint16))
+        T.prefill_attend_affine_ws(dq.ptr, B, H, Hkv, L, D, 64, 4, 4, D ** -0.5, [seg], out.ptr,
+                                   ws.ptr, ws_bytes, q_start, 0, causal, window)
+        T.hip().sync()
+        assert np.array_equal(out.numpy(), got["0"]), f"workspace of {ws_bytes} bytes"
+
+
 @pytest.mark.parametrize("case", [0, 1, 3, 4, 5, 7, 9, 10, 12, 13])
 def test_prefill_dequantize_once_is_bit_identical(T, monkeypatch, case):
     # Keys dequantized once into scratch (mlx::dequantize's bits) and then
