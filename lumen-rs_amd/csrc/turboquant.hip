@@ -1,6 +1,7 @@
 // TurboQuant codebook format on the device: encode (rotate, normalize,
-// Lloyd-Max codes, QJL residual signs), the SimpleCache estimators, rotation,
-// and fused decode attention over codebook caches.
+// Lloyd-Max codes, QJL residual signs), the SimpleCache estimators and the
+// rotation. (The GPU path's encode is tq_encode_gpu.hip, decode attention over
+// codebook caches codebook_decode.hip.)
 //
 // The encode and the estimators are bit-exact restatements of lumen-core's
 // CPU path, so codes, scales, signs and scores equal the reference's given
@@ -930,426 +931,6 @@ extern "C" int32_t tqkv_rotate_bf16(const uint16_t* x, int64_t rows, int32_t dim
   return ok();
 }
 
-// ---------------------------------------------------------------------------
-// Decode attention over a codebook cache (the GPU TurboQuant caches'
-// fused attention, turboquant.rs:763-923, for one query position): keys and
-// values are stored rotated (y = R x) as codes + sigma, so the query is
-// rotated the same way, attention runs in the rotated basis over
-// centroid[c] * sigma, and the output goes back through R^T.
-namespace tqkv {
-namespace tq {
-namespace {
-
-constexpr int kCbTile = 64;  // tokens per step of a wavefront
-
-// q_rot[b, h, :] = R q[b, h, :] in f32, and qs = q_rot * qscale (the
-// scores' query). A workgroup takes kRotRows (batch row, head) rows and 64
-// outputs (blockIdx.y); a wavefront takes four outputs at a time for all
-// its rows: its lanes read rows i of R (coalesced) against the queries,
-// then sum across the lanes. Each load of R serves kRotRows rows (a
-// workgroup a row, reading all of R, made 128 MiB of L2 reads at config
-// 2's shape). Every output's sum runs in the same order either way.
-// blockDim: 256 (4 wavefronts x 4 outputs x 4 steps = 64 outputs).
-constexpr int kRotRows = 4;
-__global__ __launch_bounds__(256) void cb_rotate_q_kernel(const uint16_t* __restrict__ q,
-                                                          const float* __restrict__ R, int D,
-                                                          int64_t rows, float qscale,
-                                                          float* __restrict__ qr,
-                                                          float* __restrict__ qs) {
-  const int64_t r0 = int64_t(blockIdx.x) * kRotRows;
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const uint16_t* qrow[kRotRows];
-#pragma unroll
-  for (int k = 0; k < kRotRows; ++k)
-    qrow[k] = q + (r0 + k < rows ? r0 + k : rows - 1) * D;  // rows past the end repeat one
-  for (int i0 = int(blockIdx.y) * kWave + 4 * wave; i0 < (int(blockIdx.y) + 1) * kWave;
-       i0 += 16) {
-    float acc[kRotRows][4] = {};
-    for (int j = lane; j < D; j += kWave) {
-      float x[kRotRows];
-#pragma unroll
-      for (int k = 0; k < kRotRows; ++k) x[k] = bf16_to_f32(qrow[k][j]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float rv = R[int64_t(i0 + r) * D + j];
-#pragma unroll
-        for (int k = 0; k < kRotRows; ++k) acc[k][r] = fmaf(rv, x[k], acc[k][r]);
-      }
-    }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1)
-#pragma unroll
-      for (int k = 0; k < kRotRows; ++k)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[k][r] += __shfl_xor(acc[k][r], off, kWave);
-#pragma unroll
-    for (int k = 0; k < kRotRows; ++k) {
-      if (lane < 4 && r0 + k < rows) {
-        const float v =
-            lane == 0 ? acc[k][0] : lane == 1 ? acc[k][1] : lane == 2 ? acc[k][2] : acc[k][3];
-        qr[(r0 + k) * D + i0 + lane] = v;
-        qs[(r0 + k) * D + i0 + lane] = v * qscale;
-      }
-    }
-  }
-}
-
-// pq = Phi q for every (batch row, head): the query's QJL projection
-// (QJLProjector::project_query, qjl.rs:76-84) for the score correction.
-__global__ void cb_project_q_kernel(const uint16_t* __restrict__ q, const float* __restrict__ phi,
-                                    int D, int m, float* __restrict__ pq) {
-  const int64_t bh = blockIdx.x;
-  for (int row = threadIdx.x; row < m; row += blockDim.x) {
-    float acc = 0.0f;
-    for (int j = 0; j < D; ++j) acc = fmaf(phi[int64_t(row) * D + j], bf16_to_f32(q[bh * D + j]), acc);
-    pq[bh * m + row] = acc;
-  }
-}
-
-// pq = Phi (R_eff q) from the rotated f32 query: the QJL projection of a
-// cache whose signs are of the rotated-basis residual (the GPU-path encode).
-__global__ void cb_project_qr_kernel(const float* __restrict__ qr, const float* __restrict__ phi,
-                                     int D, int m, float* __restrict__ pq) {
-  const int64_t bh = blockIdx.x;
-  for (int row = threadIdx.x; row < m; row += blockDim.x) {
-    float acc = 0.0f;
-    for (int j = 0; j < D; ++j) acc = fmaf(phi[int64_t(row) * D + j], qr[bh * D + j], acc);
-    pq[bh * m + row] = acc;
-  }
-}
-
-// Most QJL rows the fused decode takes (m = 32 * qjl_words).
-constexpr int kMaxQjl = 1024;
-
-// One workgroup of one wavefront per (split, KV head, batch row): partial
-// softmax state over its tokens for the G query heads. Scores: lane = token;
-// values: lane = D / 64 consecutive channels. QJL: each key's score gains the
-// QJL estimate of q . r from its residual signs (estimate_correction,
-// qjl.rs:86-118; the two-stage scores of compressor.rs:122-159), with the
-// query's projection in LDS.
-template <int D, int G, bool QJL>
-__global__ __launch_bounds__(kWave) void cb_decode_kernel(
-    const float* __restrict__ qs, int H, const uint8_t* __restrict__ kc,
-    const float* __restrict__ ks, const uint8_t* __restrict__ vc, const float* __restrict__ vs,
-    int64_t cap, int64_t n, int H_kv, const float* __restrict__ cent_k,
-    const float* __restrict__ cent_v, int n_k, int n_v, float qscale, int64_t split_len,
-    int n_splits, float* __restrict__ part_o, float* __restrict__ part_m,
-    float* __restrict__ part_l, const uint32_t* __restrict__ ksg, const float* __restrict__ krn,
-    const float* __restrict__ pq, int qm, int hg) {
-  constexpr int PER = D / kWave;
-  __shared__ float s_ck[256], s_cv[256];
-  __shared__ float s_p[G][kCbTile];
-  __shared__ float s_pq[QJL ? G : 1][QJL ? kMaxQjl : 1];
-  // blockIdx.y: KV head x head group (hg groups of G query heads each).
-  const int split = blockIdx.x, b = blockIdx.z;
-  const int kvh = int(blockIdx.y) / hg;
-  const int h0 = kvh * G * hg + (int(blockIdx.y) % hg) * G;  // first query head
-  const int lane = threadIdx.x;
-  // The scaled query of the G heads: every lane reads the same values, so
-  // the compiler loads them into scalar registers (s_load) as the scores
-  // need them, where copies in LDS took a vector LDS read per four values
-  // (measured at config 2's shape: 1.026 -> 0.960 ms a call).
-  const float* qg = qs + (int64_t(b) * H + h0) * D;
-  if constexpr (QJL) {
-    for (int i = lane; i < G * qm; i += kWave) {
-      const int h = i / qm, r = i % qm;
-      s_pq[h][r] = pq[(int64_t(b) * H + h0 + h) * qm + r];
-    }
-  }
-  for (int i = lane; i < 256; i += kWave) {
-    s_ck[i] = i < n_k ? cent_k[i] : 0.0f;
-    s_cv[i] = i < n_v ? cent_v[i] : 0.0f;
-  }
-  __syncthreads();
-  const int64_t slab = (int64_t(b) * H_kv + kvh) * cap;
-  const int64_t t0 = int64_t(split) * split_len;
-  const int64_t t1 = t0 + split_len < n ? t0 + split_len : n;
-  float m[G], l[G], acc[G][PER];
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
-    m[h] = -INFINITY;
-    l[h] = 0.0f;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) acc[h][k] = 0.0f;
-  }
-  // D <= 256: the lane's key row of the next tile loads while this tile's
-  // softmax and values run (16 B a load, D / 16 registers of 4 words).
-  // D = 256 (kVRegs): once a tile's keys are scored, their 64 registers take
-  // the tile's 64 value words (one 4-byte load a token, all issued at once,
-  // landing under the softmax), and the next tile's key row loads a quarter
-  // at a time as the value words are used up. A value loop that loaded
-  // words as it went waited for memory every four tokens.
-  constexpr bool kAhead = D <= 256;
-  constexpr bool kVRegs = D == 256;
-  constexpr int KW = kAhead ? D / 16 : 1;
-  // The scores' loop over a key row: whole at D <= 256 (the row is in
-  // registers); at D = 512, eight 16-byte loads in flight (unrolled by one,
-  // each load had waited for the last).
-  constexpr int KU = kAhead ? KW : 8;
-  uint4 kn[KW];
-  // Unconditional loads (a lane past the range re-reads the range's last
-  // row, whose scores it masks): a lane that kept its old row instead would
-  // hold both rows' registers live at once.
-  auto load_keys_part = [&](int64_t at, int i0, int i1) {
-    const uint8_t* row = kc + (slab + (at < t1 ? at : t1 - 1)) * D;
-#pragma unroll
-    for (int i = i0; i < i1; ++i) kn[i] = *reinterpret_cast<const uint4*>(row + 16 * i);
-  };
-  auto load_keys = [&](int64_t at) { load_keys_part(at, 0, KW); };
-  if constexpr (kAhead) load_keys(t0 + lane);
-  for (int64_t base = t0; base < t1; base += kCbTile) {
-    const int64_t t = base + lane;
-    const bool valid = t < t1;
-    float sc[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) sc[h] = 0.0f;
-    if (valid) {
-      const uint8_t* row = kc + (slab + t) * D;
-#pragma unroll KU
-      for (int d = 0; d < D; d += 16) {
-        const uint4 w = kAhead ? kn[d / 16] : *reinterpret_cast<const uint4*>(row + d);
-        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          const float c = s_ck[(ws[k / 4] >> (8 * (k % 4))) & 0xffu];
-#pragma unroll
-          for (int h = 0; h < G; ++h) sc[h] = fmaf(qg[h * D + d + k], c, sc[h]);
-        }
-      }
-      const float sg = ks[slab + t];
-#pragma unroll
-      for (int h = 0; h < G; ++h) sc[h] *= sg;
-      if constexpr (QJL) {
-        const float rn = krn[slab + t];
-        if (rn >= 1e-10f) {
-          const int words = (qm + 31) / 32;
-          const uint32_t* sw = ksg + (slab + t) * words;
-          float corr[G];
-#pragma unroll
-          for (int h = 0; h < G; ++h) corr[h] = 0.0f;
-          for (int w = 0; w < words; ++w) {
-            const uint32_t bits = sw[w];
-            const int nb = qm - 32 * w < 32 ? qm - 32 * w : 32;
-            for (int j = 0; j < nb; ++j) {
-              const bool pos = (bits >> j) & 1u;
-#pragma unroll
-              for (int h = 0; h < G; ++h) {
-                const float p = s_pq[h][32 * w + j];
-                corr[h] += pos ? p : -p;
-              }
-            }
-          }
-          const float cm = rn * (1.2533141373155001f / sqrtf(float(qm)));  // sqrt(pi/2) / sqrt(m)
-#pragma unroll
-          for (int h = 0; h < G; ++h) sc[h] = fmaf(corr[h] * cm, qscale, sc[h]);
-        }
-      }
-    }
-    const int cnt = int(t1 - base < kCbTile ? t1 - base : kCbTile);
-    uint32_t vw[kVRegs ? kCbTile : 1];
-    const uint8_t* vrow = vc + (slab + base) * D + PER * lane;
-    if constexpr (kVRegs) {
-      // Tokens past the range re-read the last row; their weights are 0.
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < kCbTile; ++j)
-        vw[j] = *reinterpret_cast<const uint32_t*>(vrow + int64_t(j < cnt ? j : cnt - 1) * D);
-    } else if constexpr (kAhead) {
-      load_keys(t + kCbTile);  // this tile's keys are scored
-    }
-    // D < 256: the values' codes go through registers 16 tokens at a time,
-    // two groups in flight (the first two load under the softmax), in
-    // place of a loop that loaded each token's codes as it went.
-    constexpr bool kVGroups = D < 256;
-    constexpr int VWD = (PER + 3) / 4;  // words of a lane's codes a token
-    constexpr int NGT = 16;             // tokens a group
-    uint32_t va[kVGroups ? NGT : 1][VWD], vb[kVGroups ? NGT : 1][VWD];
-    auto load_group = [&](uint32_t (&dst)[kVGroups ? NGT : 1][VWD], int g) {
-#pragma unroll
-      for (int u = 0; u < NGT; ++u) {
-        const int j = g * NGT + u;
-        const uint8_t* src = vrow + int64_t(j < cnt ? j : cnt - 1) * D;
-        if constexpr (PER == 1) {
-          dst[u][0] = *src;
-        } else if constexpr (PER == 2) {
-          dst[u][0] = *reinterpret_cast<const uint16_t*>(src);
-        } else {
-#pragma unroll
-          for (int w = 0; w < VWD; ++w) dst[u][w] = *reinterpret_cast<const uint32_t*>(src + 4 * w);
-        }
-      }
-    };
-    auto use_group = [&](const uint32_t (&src)[kVGroups ? NGT : 1][VWD], int g) {
-#pragma unroll
-      for (int u = 0; u < NGT; ++u) {
-        const int j = g * NGT + u;
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-          const float c = s_cv[(src[u][k / 4] >> (8 * (k % 4))) & 0xffu];
-#pragma unroll
-          for (int h = 0; h < G; ++h) acc[h][k] = fmaf(s_p[h][j], c, acc[h][k]);
-        }
-      }
-    };
-    if constexpr (kVGroups) {
-      load_group(va, 0);
-      load_group(vb, 1);
-    }
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float mx = valid ? sc[h] : -INFINITY;
-#pragma unroll
-      for (int off = 1; off < kWave; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-      const float mn = fmaxf(m[h], mx);
-      const float f = m[h] == -INFINITY ? 0.0f : exp2f(m[h] - mn);
-      l[h] *= f;
-#pragma unroll
-      for (int k = 0; k < PER; ++k) acc[h][k] *= f;
-      m[h] = mn;
-      const float p = valid ? exp2f(sc[h] - mn) : 0.0f;
-      float ps = p;
-#pragma unroll
-      for (int off = 1; off < kWave; off <<= 1) ps += __shfl_xor(ps, off, kWave);
-      l[h] += ps;
-      s_p[h][lane] = valid ? p * vs[slab + t] : 0.0f;
-    }
-    __syncthreads();
-    // Values: lane takes channels PER * lane .. + PER - 1 (one PER-byte load
-    // of each token's row; the wavefront reads the row whole).
-    if constexpr (kVRegs) {
-#pragma unroll
-      for (int qq = 0; qq < 4; ++qq) {
-#pragma unroll
-        for (int j = 16 * qq; j < 16 * qq + 16; ++j) {
-#pragma unroll
-          for (int k = 0; k < PER; ++k) {
-            const float c = s_cv[(vw[j] >> (8 * k)) & 0xffu];
-#pragma unroll
-            for (int h = 0; h < G; ++h) acc[h][k] = fmaf(s_p[h][j], c, acc[h][k]);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        load_keys_part(t + kCbTile, qq * (KW / 4), (qq + 1) * (KW / 4));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    if constexpr (kVGroups) {
-      // Tokens past the range re-read the last row; their weights are 0.
-      use_group(va, 0);
-      load_group(va, 2);
-      use_group(vb, 1);
-      load_group(vb, 3);
-      use_group(va, 2);
-      use_group(vb, 3);
-    }
-    // D = 512: one token's codes at a time (two words a lane; staged
-    // groups measured slower at Gemma 4's global shape).
-    for (int j = 0; j < (D > 256 ? cnt : 0); ++j) {
-      uint32_t cw[VWD];
-#pragma unroll
-      for (int w = 0; w < VWD; ++w)
-        cw[w] = *reinterpret_cast<const uint32_t*>(vrow + int64_t(j) * D + 4 * w);
-#pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const float c = s_cv[(cw[k / 4] >> (8 * (k % 4))) & 0xffu];
-#pragma unroll
-        for (int h = 0; h < G; ++h) acc[h][k] = fmaf(s_p[h][j], c, acc[h][k]);
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
-    const int64_t row = (int64_t(b) * H + h0 + h) * n_splits + split;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) part_o[row * D + PER * lane + k] = acc[h][k];
-    if (lane == 0) {
-      part_m[row] = m[h];
-      part_l[row] = l[h];
-    }
-  }
-}
-
-// Merge the splits of one (batch row, head) in the rotated basis, then
-// o = R^T o_rot, as bf16.
-__global__ void cb_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_m,
-                                const float* __restrict__ part_l, int n_splits, int D,
-                                const float* __restrict__ R, uint16_t* __restrict__ out) {
-  extern __shared__ float s_o[];
-  const int64_t bh = blockIdx.x;
-  const float* pm = part_m + bh * n_splits;
-  const float* pl = part_l + bh * n_splits;
-  float mx = -INFINITY;
-  for (int s = 0; s < n_splits; ++s) mx = fmaxf(mx, pm[s]);
-  // Each split's weight once (the same exp2f of the same argument as a
-  // per-element evaluation; empty splits are skipped by their max).
-  float* s_w = s_o + D;
-  for (int s = threadIdx.x; s < n_splits; s += blockDim.x)
-    s_w[s] = pm[s] != -INFINITY ? exp2f(pm[s] - mx) : 0.0f;
-  __syncthreads();
-  // No branch per split (an empty split's weight is 0, and the decode
-  // writes its partial as zeros), so the unrolled loads issue together: a
-  // test per split had them wait one at a time.
-  float ls = 0.0f;
-  for (int s = 0; s < n_splits; ++s) ls += pl[s] * s_w[s];
-  for (int d = threadIdx.x; d < D; d += blockDim.x) {
-    float os = 0.0f;
-#pragma unroll 16
-    for (int s = 0; s < n_splits; ++s) os += part_o[(bh * n_splits + s) * D + d] * s_w[s];
-    s_o[d] = ls > 0.0f ? os / ls : 0.0f;
-  }
-  __syncthreads();
-  // o = R^T o_rot: a thread's outputs (one, or two at D = 512) in one loop,
-  // sixteen steps of loads of R in flight (the sums' order per output is
-  // the sequence j = 0 .. D-1 either way).
-  const int i0 = threadIdx.x, i1 = threadIdx.x + blockDim.x;
-  const bool two = i1 < D;
-  float a0 = 0.0f, a1 = 0.0f;
-  if (two) {
-#pragma unroll 16
-    for (int j = 0; j < D; ++j) {
-      const float o = s_o[j];
-      a0 = fmaf(R[int64_t(j) * D + i0], o, a0);
-      a1 = fmaf(R[int64_t(j) * D + i1], o, a1);
-    }
-  } else {
-#pragma unroll 16
-    for (int j = 0; j < D; ++j) a0 = fmaf(R[int64_t(j) * D + i0], s_o[j], a0);
-  }
-  if (i0 < D) out[bh * D + i0] = f32_to_bf16(a0);
-  if (two) out[bh * D + i1] = f32_to_bf16(a1);
-}
-
-template <int D>
-int32_t launch_cb(int G, dim3 grid, hipStream_t st, const float* qs, int H, const uint8_t* kc,
-                  const float* ks, const uint8_t* vc, const float* vs, int64_t cap, int64_t n,
-                  int H_kv, const float* ck, const float* cv, int nk, int nv, float qscale,
-                  int64_t split_len, int n_splits, float* po, float* pm, float* pl,
-                  const uint32_t* ksg, const float* krn, const float* pq, int m, int hg) {
-#define TQKV_CB(GG)                                                                           \
-  case GG:                                                                                   \
-    if (ksg)                                                                                 \
-      hipLaunchKernelGGL((cb_decode_kernel<D, GG, true>), grid, dim3(kWave), 0, st, qs, H, kc, \
-                         ks, vc, vs, cap, n, H_kv, ck, cv, nk, nv, qscale, split_len, n_splits, \
-                         po, pm, pl, ksg, krn, pq, m, hg);                                    \
-    else                                                                                     \
-      hipLaunchKernelGGL((cb_decode_kernel<D, GG, false>), grid, dim3(kWave), 0, st, qs, H, kc,\
-                         ks, vc, vs, cap, n, H_kv, ck, cv, nk, nv, qscale, split_len, n_splits, \
-                         po, pm, pl, ksg, krn, pq, m, hg);                                    \
-    break;
-  switch (G) {
-    TQKV_CB(1) TQKV_CB(2) TQKV_CB(4) TQKV_CB(8) TQKV_CB(16)
-    default: return fail(TQKV_EUNSUPPORTED, "codebook decode with %d query heads a wavefront", G);
-  }
-#undef TQKV_CB
-  TQKV_LAUNCHED();
-  return TQKV_OK;
-}
-
-}  // namespace
-}  // namespace tq
-}  // namespace tqkv
-
 namespace tqkv {
 namespace tq {
 namespace {
@@ -1419,158 +1000,4 @@ extern "C" int32_t tqkv_codebook_dequantize(const uint8_t* codes, const float* s
                                                    dim, out, reinterpret_cast<hipStream_t>(stream)))
     return rc;
   return ok();
-}
-
-extern "C" size_t tqkv_decode_codebook_workspace_size(int32_t B, int32_t H, int32_t D,
-                                                       int64_t total_tokens) {
-  if (B <= 0 || H <= 0 || D <= 0 || total_tokens <= 0) return 0;
-  // The most splits decode_codebook plans for any context up to total_tokens.
-  const int64_t splits = (total_tokens + 255) / 256 < 64 ? (total_tokens + 255) / 256 : 64;
-  return size_t(B) * H *
-         (2 * size_t(D) + size_t(tq::kMaxQjl) + size_t(splits) * (size_t(D) + 2)) * sizeof(float);
-}
-
-namespace {
-int32_t decode_codebook(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, int32_t D,
-                        float scale, const float* rotation, const float* centroids_k,
-                        int32_t bits_k, const float* centroids_v, int32_t bits_v,
-                        const uint8_t* k_codes, const float* k_sigma, const uint32_t* k_signs,
-                        const float* k_rnorm, const float* qjl, int32_t qjl_m,
-                        const uint8_t* v_codes, const float* v_sigma, int64_t cap, int64_t n,
-                        uint16_t* out, void* workspace, size_t workspace_bytes,
-                        tqkv_stream stream, bool qjl_rotated = false) {
-  if (!q || !rotation || !centroids_k || !centroids_v || !k_codes || !k_sigma || !v_codes ||
-      !v_sigma || !out)
-    return fail(TQKV_EINVAL_ARG, "null pointer");
-  if (qjl_m != 0 && (!k_signs || !k_rnorm || !qjl || qjl_m < 0 || qjl_m > tq::kMaxQjl))
-    return fail(TQKV_EINVAL_ARG, "qjl_m=%d needs signs, residual norms and the QJL matrix "
-                "(m <= %d)", qjl_m, tq::kMaxQjl);
-  if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || n <= 0 || n > cap)
-    return fail(TQKV_EINVAL_SHAPE, "B=%d H=%d H_kv=%d n=%lld cap=%lld", B, H, H_kv, (long long)n,
-                (long long)cap);
-  if (bits_k < 1 || bits_k > 8 || bits_v < 1 || bits_v > 8)
-    return fail(TQKV_EUNSUPPORTED, "bits %d/%d", bits_k, bits_v);
-  // A lane loads D / 64 value codes at once (up to 4-byte words); key rows
-  // are read 16 bytes a load (rows of D >= 64 bytes keep that alignment).
-  const int v_align = D >= 256 ? 4 : D >= 128 ? 2 : 1;
-  if (reinterpret_cast<uintptr_t>(v_codes) % v_align != 0)
-    return fail(TQKV_EINVAL_ARG, "v_codes must be %d-byte aligned", v_align);
-  if (reinterpret_cast<uintptr_t>(k_codes) % 16 != 0)
-    return fail(TQKV_EINVAL_ARG, "k_codes must be 16-byte aligned");
-  const int G = H / H_kv;
-  if (G > 16 || (G & (G - 1)) != 0)
-    return fail(TQKV_EUNSUPPORTED, "codebook decode with %d query heads per KV head (1, 2, 4, "
-                "8 or 16)", G);
-  // A wavefront takes Gw = G / hg of a KV head's query heads, Gw x D <= 1024
-  // (each head group re-reads the keys and values, mostly from L2): at D =
-  // 512 with 16 heads a KV head (Gemma 4's global layers) one wavefront of
-  // all 16 heads held 251 registers and the few (batch row, KV head) units
-  // left most SIMDs idle.
-  int hg = 1;
-  while (G / hg > 1 && (G / hg) * D > 1024) hg *= 2;
-  const int Gw = G / hg;
-  // Splits: with 128 or more (batch row, KV head, head group) units the grid
-  // fills the chip with splits of 1024 tokens (at most 32), which pay the
-  // first key load and the merge half as often (config 2's shape: 1.061
-  // against 1.094 ms); fewer units take enough splits for ~4,096
-  // wavefronts, never under 256 tokens a split, at most 64 (the workspace
-  // size assumes no more).
-  const int64_t units = int64_t(B) * H_kv * hg;
-  int64_t n_splits64;
-  if (units >= 128) {
-    n_splits64 = (n + 1023) / 1024 < 32 ? (n + 1023) / 1024 : 32;
-  } else {
-    n_splits64 = (4096 + units - 1) / units;
-    if (n_splits64 > (n + 255) / 256) n_splits64 = (n + 255) / 256;
-    if (n_splits64 > 64) n_splits64 = 64;
-  }
-  const int n_splits = int(n_splits64);
-  const int64_t split_len = (n + n_splits - 1) / n_splits;
-  const size_t need = tqkv_decode_codebook_workspace_size(B, H, D, n);
-  void* ws = workspace;
-  if (!ws) {
-    if (int32_t rc = scratch_for_current_device(need, &ws)) return rc;
-  } else if (workspace_bytes < need) {
-    return fail(TQKV_EINVAL_ARG, "workspace of %zu bytes, need %zu", workspace_bytes, need);
-  }
-  float* qr = static_cast<float*>(ws);
-  float* qsc = qr + size_t(B) * H * D;
-  float* pq = qsc + size_t(B) * H * D;
-  float* po = pq + size_t(B) * H * tq::kMaxQjl;
-  float* pm = po + size_t(B) * H * n_splits * D;
-  float* pl = pm + size_t(B) * H * n_splits;
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const float qscale = scale * 1.4426950408889634f;
-  const int64_t qrows = int64_t(B) * H;
-  hipLaunchKernelGGL(tq::cb_rotate_q_kernel,
-                     dim3(unsigned((qrows + tq::kRotRows - 1) / tq::kRotRows), unsigned(D / 64)),
-                     dim3(256), 0, st, q, rotation, D, qrows, qscale, qr, qsc);
-  TQKV_LAUNCHED();
-  if (qjl_m > 0) {
-    if (qjl_rotated)
-      hipLaunchKernelGGL(tq::cb_project_qr_kernel, dim3(unsigned(B * H)), dim3(256), 0, st, qr,
-                         qjl, D, qjl_m, pq);
-    else
-      hipLaunchKernelGGL(tq::cb_project_q_kernel, dim3(unsigned(B * H)), dim3(256), 0, st, q,
-                         qjl, D, qjl_m, pq);
-    TQKV_LAUNCHED();
-  }
-  const uint32_t* sg = qjl_m > 0 ? k_signs : nullptr;
-  const dim3 grid{unsigned(n_splits), unsigned(H_kv * hg), unsigned(B)};
-  int32_t rc = TQKV_OK;
-  switch (D) {
-    case 64: rc = tq::launch_cb<64>(Gw, grid, st, qsc, H, k_codes, k_sigma, v_codes, v_sigma, cap, n, H_kv, centroids_k, centroids_v, 1 << bits_k, 1 << bits_v, qscale, split_len, n_splits, po, pm, pl, sg, k_rnorm, pq, qjl_m, hg); break;
-    case 128: rc = tq::launch_cb<128>(Gw, grid, st, qsc, H, k_codes, k_sigma, v_codes, v_sigma, cap, n, H_kv, centroids_k, centroids_v, 1 << bits_k, 1 << bits_v, qscale, split_len, n_splits, po, pm, pl, sg, k_rnorm, pq, qjl_m, hg); break;
-    case 256: rc = tq::launch_cb<256>(Gw, grid, st, qsc, H, k_codes, k_sigma, v_codes, v_sigma, cap, n, H_kv, centroids_k, centroids_v, 1 << bits_k, 1 << bits_v, qscale, split_len, n_splits, po, pm, pl, sg, k_rnorm, pq, qjl_m, hg); break;
-    case 512: rc = tq::launch_cb<512>(Gw, grid, st, qsc, H, k_codes, k_sigma, v_codes, v_sigma, cap, n, H_kv, centroids_k, centroids_v, 1 << bits_k, 1 << bits_v, qscale, split_len, n_splits, po, pm, pl, sg, k_rnorm, pq, qjl_m, hg); break;
-    default: return fail(TQKV_EUNSUPPORTED, "codebook decode D=%d not in {64,128,256,512}", D);
-  }
-  if (rc) return rc;
-  hipLaunchKernelGGL(tq::cb_merge_kernel, dim3(unsigned(B * H)), dim3(D < 256 ? D : 256),
-                     size_t(D + n_splits) * sizeof(float), st, po, pm, pl, n_splits, D, rotation,
-                     out);
-  TQKV_LAUNCHED();
-  return ok();
-}
-}  // namespace
-
-extern "C" int32_t tqkv_decode_attend_codebook(
-    const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, int32_t D, float scale,
-    const float* rotation, const float* centroids_k, int32_t bits_k, const float* centroids_v,
-    int32_t bits_v, const uint8_t* k_codes, const float* k_sigma, const uint8_t* v_codes,
-    const float* v_sigma, int64_t cap, int64_t n, uint16_t* out, void* workspace,
-    size_t workspace_bytes, tqkv_stream stream) {
-  return decode_codebook(q, B, H, H_kv, D, scale, rotation, centroids_k, bits_k, centroids_v,
-                         bits_v, k_codes, k_sigma, nullptr, nullptr, nullptr, 0, v_codes, v_sigma,
-                         cap, n, out, workspace, workspace_bytes, stream);
-}
-
-namespace tqkv {
-// Codebook decode with QJL signs of the rotated-basis residual (a GPU-path
-// cache): the score correction projects the rotated query.
-int32_t decode_codebook_qjl_rotated(
-    const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, int32_t D, float scale,
-    const float* rotation, const float* centroids_k, int32_t bits_k, const float* centroids_v,
-    int32_t bits_v, const uint8_t* k_codes, const float* k_sigma, const uint32_t* k_signs,
-    const float* k_rnorm, const float* qjl, int32_t qjl_m, const uint8_t* v_codes,
-    const float* v_sigma, int64_t cap, int64_t n, uint16_t* out, void* workspace,
-    size_t workspace_bytes, tqkv_stream stream) {
-  if (qjl_m <= 0) return fail(TQKV_EINVAL_ARG, "qjl_m=%d", qjl_m);
-  return decode_codebook(q, B, H, H_kv, D, scale, rotation, centroids_k, bits_k, centroids_v,
-                         bits_v, k_codes, k_sigma, k_signs, k_rnorm, qjl, qjl_m, v_codes, v_sigma,
-                         cap, n, out, workspace, workspace_bytes, stream, true);
-}
-}  // namespace tqkv
-
-extern "C" int32_t tqkv_decode_attend_codebook_qjl(
-    const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, int32_t D, float scale,
-    const float* rotation, const float* centroids_k, int32_t bits_k, const float* centroids_v,
-    int32_t bits_v, const uint8_t* k_codes, const float* k_sigma, const uint32_t* k_signs,
-    const float* k_rnorm, const float* qjl, int32_t qjl_m, const uint8_t* v_codes,
-    const float* v_sigma, int64_t cap, int64_t n, uint16_t* out, void* workspace,
-    size_t workspace_bytes, tqkv_stream stream) {
-  if (qjl_m <= 0) return fail(TQKV_EINVAL_ARG, "qjl_m=%d", qjl_m);
-  return decode_codebook(q, B, H, H_kv, D, scale, rotation, centroids_k, bits_k, centroids_v,
-                         bits_v, k_codes, k_sigma, k_signs, k_rnorm, qjl, qjl_m, v_codes, v_sigma,
-                         cap, n, out, workspace, workspace_bytes, stream);
 }

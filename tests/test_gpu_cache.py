@@ -374,6 +374,72 @@ def test_codebook_decode_direct(T, B, Hkv, G, D, N, bits):
     check_bf16(out.numpy().reshape(B, H, D), want, f"codebook-direct B={B} Hkv={Hkv} D={D}")
 
 
+@pytest.mark.parametrize("D,G,N,bits_k,bits_v,m,mag", [
+    (64, 1, 1, 1, 8, 0, 0), (64, 8, 63, 4, 4, 31, 0), (64, 16, 257, 5, 3, 0, 8),
+    (128, 2, 65, 2, 2, 33, 0), (128, 4, 129, 3, 4, 0, 8), (128, 1, 700, 8, 8, 0, 0),
+    (256, 2, 64, 3, 3, 64, 0), (256, 16, 513, 4, 4, 96, 8), (256, 8, 300, 6, 4, 0, 0),
+    (512, 16, 127, 4, 4, 0, 8), (512, 4, 128, 4, 4, 1024, 0), (512, 16, 641, 7, 7, 40, 0),
+    (512, 1, 130, 1, 1, 0, 0)])
+def test_codebook_decode_tiles(T, D, G, N, bits_k, bits_v, m, mag):
+    """The decode's tile edges (64 tokens, 128 at D = 512), splits, head groups
+    (hi and lo in one operand up to 8 heads, apart at 16), paired (both
+    widths <= 4 bits) and single lookups, sign rows that are no multiple of
+    32, sigmas that grow by 10^(2 mag) along the tokens, a zero sigma and
+    centroids scaled by 10^mag, against the same attention in f64."""
+    print(f"[codebook-tiles] D={D} G={G} N={N} bits={bits_k}/{bits_v} m={m} mag={mag}", flush=True)
+    B, Hkv, cap = 2, 2, N + 3
+    H, rng = G * Hkv, np.random.default_rng(D * 7 + N)
+    q = O.bf16_from_f32(rng.standard_normal((B, H, D)).astype(np.float32))
+    R = T.rotation_matrix(D, 42)
+    ck, cv = ((10.0 ** mag * T.lloyd_max(b, 100)[1]).astype(np.float32) for b in (bits_k, bits_v))
+    kc = rng.integers(0, 1 << bits_k, (B, Hkv, cap, D), dtype=np.uint8)
+    vc = rng.integers(0, 1 << bits_v, (B, Hkv, cap, D), dtype=np.uint8)
+    ks = (10.0 ** -mag * rng.uniform(0.5, 2, (B, Hkv, cap))).astype(np.float32)
+    vs = (rng.uniform(0.5, 2, (B, Hkv, cap)) *
+          10.0 ** (-2.0 * mag * np.arange(cap)[::-1] / cap)).astype(np.float32)
+    if N > 1:  # (one token of zeros would leave nothing to scale the error by)
+        vs[..., N // 2] = 0
+    signs = rng.integers(0, 1 << 32, (B, Hkv, cap, (m + 31) // 32), dtype=np.uint32)
+    rn = rng.uniform(0, 1, (B, Hkv, cap)).astype(np.float32)
+    rn[..., 0] = 0
+    phi = (rng.standard_normal((max(m, 1), D)) / np.sqrt(max(m, 1))).astype(np.float32)
+    # Value codes one byte off where the width of a lane's load allows it.
+    off = 1 if D == 64 else 2 if D == 128 else 0
+    raw = np.zeros(vc.size + 4, np.uint8)
+    raw[off:off + vc.size] = vc.reshape(-1)
+    d = {n: T.DeviceArray.of(x) for n, x in dict(q=q, R=R, ck=ck, cv=cv, kc=kc, ks=ks, vc=raw, vs=vs,
+                                                sg=signs if m else rn, rn=rn, phi=phi).items()}
+    out = T.DeviceArray((B, H, 1, D), np.uint16)
+    wsb = T.decode_codebook_workspace_size(B, H, D, N)
+    ws = T.DeviceArray((wsb,), np.uint8)
+    head = (d["q"].ptr, B, H, Hkv, D, D ** -0.5, d["R"].ptr, d["ck"].ptr, bits_k, d["cv"].ptr, bits_v)
+    tail = (d["vc"].ptr + off, d["vs"].ptr, cap, N, out.ptr, ws.ptr, wsb, None)
+    if m:
+        T.check(T.lib().tqkv_decode_attend_codebook_qjl(*head, d["kc"].ptr, d["ks"].ptr, d["sg"].ptr,
+                                                        d["rn"].ptr, d["phi"].ptr, m, *tail))
+    else:
+        T.decode_attend_codebook(*head, d["kc"].ptr, d["ks"].ptr, *tail)
+    T.hip().sync()
+    q64, R64 = O.bf16_to_f32(q).astype(np.float64), R.astype(np.float64)
+    want = np.empty((B, H, D))
+    for b in range(B):
+        for h in range(H):
+            i = (b, h // G, slice(0, N))
+            k = ck.astype(np.float64)[kc[i]] * ks[i][:, None]
+            v = cv.astype(np.float64)[vc[i]] * vs[i][:, None].astype(np.float64)
+            s = k @ (R64 @ q64[b, h])
+            if m:
+                bit = (signs[i][:, np.arange(m) // 32] >> (np.arange(m) % 32).astype(np.uint32)) & 1
+                s = s + np.where(rn[i] >= 1e-10, rn[i], 0) * np.sqrt(np.pi / 2) / np.sqrt(m) * (
+                    (2.0 * bit - 1) @ (phi.astype(np.float64) @ q64[b, h]))
+            p = np.exp(s * D ** -0.5 - (s * D ** -0.5).max())
+            want[b, h] = R64.T @ ((p / p.sum()) @ v)
+    # Half a bf16 step of the largest output plus the f32 sums' error.
+    scale = np.abs(want).max()
+    check_bf16(out.numpy().reshape(B, H, D), want, "codebook-tiles", scale=scale, max_abs=1e-4,
+               mean_abs=1e-5)
+
+
 def test_codebook_decode_rejects_unaligned_values(T):
     """A lane loads its value codes 4 bytes at a time at D = 256: a value
     code pointer off that alignment is refused before any launch."""
