@@ -371,10 +371,14 @@ int32_t tqkv_decode_attend_codebook_qjl(const uint16_t* q, int32_t B, int32_t H,
  * Replaces dequantized_prefill_attention (gemma4_moe.rs:2382-2411): K and V
  * dequantize as mlx::dequantize does for bf16 (bf16(fma(scale, code,
  * bias)), one rounding), then attention runs with bf16 operands and f32 accumulation. When
- * 8 or more 256-row blocks share a KV head, the keys are dequantized once
- * into the library's per-device scratch (2 * B * H_kv * keys * D * 2 bytes,
- * at most 4 GiB; larger contexts dequantize in every block instead, in LDS)
- * and read from there; the two ways give the same bits. The mask is build_causal_mask_abs (native_attention.rs:
+ * 8 or more row blocks share a KV head (fewer at D = 256 and 512), the
+ * keys are dequantized once into the library's per-device scratch (2 * B *
+ * H_kv * keys * D * 2 bytes, at most 4 GiB; larger contexts dequantize in
+ * every block instead, in LDS) and read from there; the two ways give the
+ * same bits. A chunk with too few row blocks to fill the GPU over more than
+ * 1,024 keys that it can see splits the keys over workgroups, their partials
+ * in the same scratch, and merges them (f32, so apart from the unsplit sums
+ * by their rounding only). The mask is build_causal_mask_abs (native_attention.rs:
  * 545-622) in absolute positions: query row l sits at q_start + l and key k
  * (counted across both segments) at k_start + k; with causal != 0, key k is
  * visible iff k_abs <= q_abs and, when window > 0, q_abs < k_abs + window
@@ -402,7 +406,7 @@ int32_t tqkv_prefill_attend_affine(const uint16_t* q, int32_t B, int32_t H, int3
  * dequantize-once rows go into `workspace` when it holds
  * tqkv_prefill_workspace_size(B, H_kv, D, keys of both segments) bytes;
  * with less (or NULL) every block dequantizes its own tiles in LDS. Either
- * way the same bits, no library allocation, and calls with different
+ * way the same bits (the keys are never split here), no library allocation, and calls with different
  * workspaces may run concurrently. */
 int32_t tqkv_prefill_attend_affine_ws(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv,
                                       int32_t L, int32_t D, int32_t group_size, int32_t bits_k,

@@ -36,6 +36,10 @@ int32_t ok();
 // no workspace. Grown on demand (at least doubling, without waiting for
 // queued work: outgrown buffers are kept); freed by tqkv_scratch_release.
 int32_t scratch_for_current_device(size_t bytes, void** out);
+// The same for a path that a call can do without: false, and no error left,
+// where the scratch would have to grow under a stream capture (which an
+// allocation would end) or cannot.
+bool scratch_optional(size_t bytes, hipStream_t st, void** out);
 int32_t scratch_release_all();
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {

@@ -182,10 +182,53 @@ void dequantize_rows(const Args& a, int bk, int bv, int64_t slabs, bool tiled, h
 // Row blocks sharing one (batch row, KV head) from which the keys are
 // dequantized once into scratch instead of in every block: the blocks would
 // otherwise repeat the same dequantization, the kernel's VALU-bound part.
+// The wide kernel takes fewer: at D = 512 any (the in-block kernel spills;
+// 16 / 4 heads, 94 rows over 1,117 keys: 131 us in block, 44 once), at D = 256
+// half as many over 2,048 keys or more (B = 4, 16 / 8 heads, 300 rows over
+// 3,000 keys: 132 us in block, 107 once; 298 rows over 809: 35 and 42).
 constexpr int64_t kOnceBlocks = 8;
+int64_t once_blocks(int D, int64_t total) {
+  return D == 512 ? 1 : D == 256 && total >= 2048 ? 4 : kOnceBlocks;
+}
 // The scratch that path may take (bf16 K and V of every visible key); larger
 // contexts dequantize in every block instead.
 constexpr size_t kOnceMaxBytes = size_t(4) << 30;
+
+// Key splits of a chunk whose row blocks would leave CUs idle (a short chunk
+// over a long context): workgroups wanted, keys a split holds at least (a
+// split pays its partials' write and read), bytes of partials at most.
+// Measured (4-bit, without and with): 16 / 8 heads, D = 128, 64 rows over
+// 24,000 keys 569 and 42 us, 147 rows over 16,384 565 and 55; D = 256, 256
+// rows over 16,384 661 and 104; 32 / 2 heads, D = 512, 64 rows over 20,000
+// 2,700 and 134 (with the wide kernel).
+constexpr int64_t kSplitWorkgroups = 256, kSplitMinKeys = 512;
+constexpr size_t kSplitMaxBytes = size_t(1) << 30;
+
+// The splits' partials of each row (slots (row, split), row = (b L + l) H +
+// h) combined and written as bf16: four channels a thread.
+__global__ __launch_bounds__(256) void merge_splits_kernel(const Args a, int D, int64_t rows) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t r = i / (D / 4);
+  const int c = int(i % (D / 4)) * 4;
+  if (r >= rows) return;
+  const float* pm = a.part_m + r * a.n_part;
+  const float* pl = a.part_l + r * a.n_part;
+  float mx = -INFINITY;
+  for (int s = 0; s < a.n_part; ++s) mx = fmaxf(mx, pm[s]);
+  float l = 0.0f;
+  f4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+  for (int s = 0; s < a.n_part; ++s) {
+    const float f = pm[s] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(pm[s] - mx);
+    l += f * pl[s];
+    o += *reinterpret_cast<const f4_t*>(a.part_o + (r * a.n_part + s) * D + c) * f;
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  const int64_t h = r % a.H, bl = r / a.H;
+  uint16_t* dst = a.out + bl / a.L * a.qs_b + h * a.qs_h + bl % a.L * a.qs_l + c;
+  *reinterpret_cast<u32x2_t*>(dst) =
+      u32x2_t{pack_bf16(o[0] * inv, o[1] * inv), pack_bf16(o[2] * inv, o[3] * inv)};
+}
 
 }  // namespace
 }  // namespace prefill
@@ -403,10 +446,45 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
     default: rows_per_block = Shape<512, false>::kRows, threads = Shape<512, false>::kThreads; break;
   }
   const int64_t blocks = (int64_t(L) * a.G + rows_per_block - 1) / rows_per_block;
-  const int64_t grid = blocks * a.n_splits * H_kv * B;
-  if (grid > 0x7fffffff) return fail(TQKV_EINVAL_SHAPE, "grid too large");
+  if (blocks * H_kv * B > 0x7fffffff) return fail(TQKV_EINVAL_SHAPE, "grid too large");
+  // Key splits, over the keys some row can see, with the library's scratch
+  // (a caller's workspace holds the dequantized rows only).
+  const int64_t units = blocks * H_kv * B, q_rows = int64_t(B) * H * L;
+  if (library_scratch && units * 2 <= kSplitWorkgroups) {
+    int64_t lo = 0, hi = a.total - 1;
+    if (a.causal) {
+      if (q_start + L - 1 - k_start < hi) hi = q_start + L - 1 - k_start;
+      if (a.window >= 0 && q_start - a.window + 1 - k_start > lo) lo = q_start - a.window + 1 - k_start;
+    }
+    lo = lo / kTile * kTile;
+    int64_t splits = kSplitWorkgroups / units;
+    if (splits > (hi - lo) / kSplitMinKeys) splits = (hi - lo) / kSplitMinKeys;
+    if (splits >= 2 && size_t(q_rows) * size_t(splits) * (D + 2) * sizeof(float) <= kSplitMaxBytes) {
+      a.split_len = int((hi + 1 - lo + splits * kTile - 1) / (splits * kTile) * kTile);
+      a.n_splits = a.n_part = int((hi + 1 - lo + a.split_len - 1) / a.split_len);
+      a.split_lo = lo;
+    }
+  }
+  size_t part_bytes = a.n_splits > 1 ? size_t(q_rows) * a.n_splits * (D + 2) * sizeof(float) : 0;
+  const auto no_splits = [&] {
+    a.n_splits = a.n_part = 1;
+    a.split_len = int(a.total + kTile - 1) / kTile * kTile;
+    a.split_lo = 0;
+    part_bytes = 0;
+  };
   a.n_blocks = int(blocks);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  // The partials at p (16-byte aligned), and the merge after the kernel.
+  const auto use_parts = [&](Args& args, void* p) {
+    args.part_o = static_cast<float*>(p);
+    args.part_m = args.part_o + size_t(q_rows) * a.n_splits * D;
+    args.part_l = args.part_m + size_t(q_rows) * a.n_splits;
+  };
+  const auto merge = [&](const Args& args) {
+    const int64_t threads = q_rows * (D / 4);
+    hipLaunchKernelGGL(merge_splits_kernel, dim3(unsigned((threads + 255) / 256)), dim3(256), 0, st,
+                       args, D, q_rows);
+  };
   // TQKV_PREFILL_DEQUANT_ONCE=0 / 1 forces the choice (tests compare them).
   const char* once_env = getenv("TQKV_PREFILL_DEQUANT_ONCE");
   const int64_t slabs = int64_t(B) * H_kv;
@@ -421,14 +499,27 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   // With a caller workspace (the _ws entry) the dequantized rows go there
   // when it holds them, else every block dequantizes for itself.
   const bool fits = library_scratch || (workspace && workspace_bytes >= need);
-  const bool once = !bf16_rows && fits &&
-                    (once_env ? strcmp(once_env, "0") != 0
-                              : blocks >= kOnceBlocks &&
-                                    once_bytes(slabs, a.total, D) <= kOnceMaxBytes);
+  bool once = !bf16_rows && fits &&
+              (once_env ? strcmp(once_env, "0") != 0
+                        : blocks >= once_blocks(D, a.total) &&
+                              once_bytes(slabs, a.total, D) <= kOnceMaxBytes);
+  // Scratch that the call could do without (the partials; the rows of few
+  // blocks) is left out where the library's cannot grow.
+  void* ws = workspace;
+  if (library_scratch && (once || part_bytes)) {
+    const size_t rows_bytes = once ? need : 0;
+    bool held = part_bytes && scratch_optional(rows_bytes + part_bytes, st, &ws);
+    if (!held) no_splits();
+    if (once && !held) {
+      if (blocks >= kOnceBlocks || once_env) {
+        if (int32_t rc = scratch_for_current_device(need, &ws)) return rc;
+      } else {
+        once = scratch_optional(need, st, &ws);
+      }
+    }
+  }
+  const int64_t grid = units * a.n_splits;
   if (once) {
-    void* ws = workspace;
-    if (library_scratch)
-      if (int32_t rc = scratch_for_current_device(need, &ws)) return rc;
     uint16_t* kd = static_cast<uint16_t*>(ws);
     uint16_t* vd = kd + size_t(slabs) * size_t(slab_rows) * size_t(D);
     if (slabs > 65535) return fail(TQKV_EINVAL_SHAPE, "B * H_kv = %lld slabs", (long long)slabs);
@@ -446,24 +537,37 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
                    int64_t(H_kv) * slab_rows};
     p.seg[1] = p.seg[0];
     p.n0 = a.total;
+    if (part_bytes) use_parts(p, static_cast<char*>(ws) + need);
     if (D >= 256 && tiled) {
-      // 64-row blocks where 128-row ones would not give every CU a workgroup
-      // (32 / 2 heads, D = 512, 512 rows over 8,192 keys: 380 us with 128
-      // rows, 331 with 64).
-      const int64_t q_rows = int64_t(L) * a.G;
-      const int wide_rows = (q_rows + 127) / 128 * H_kv * B >= 256 ? 128 : 64;
-      p.n_blocks = int((q_rows + wide_rows - 1) / wide_rows);
-      hipLaunchKernelGGL(pick_wide(D, wide_rows), dim3(unsigned(p.n_blocks * int64_t(H_kv) * B)),
+      // Rows a block by rounds of workgroups over the CUs (one a CU), a 64-row
+      // block's taking 0.87 of a 128-row one's time (32 / 2 heads, D = 512,
+      // 512 rows over 8,192 keys, one round each: 331 and 380 us).
+      const int64_t unit_rows = int64_t(L) * a.G, per_block = int64_t(H_kv) * B * a.n_splits;
+      const auto rounds = [&](int64_t rows) {
+        return ((unit_rows + rows - 1) / rows * per_block + 255) / 256;
+      };
+      const int wide_rows = 100 * rounds(128) <= 87 * rounds(64) ? 128 : 64;
+      p.n_blocks = int((unit_rows + wide_rows - 1) / wide_rows);
+      hipLaunchKernelGGL(pick_wide(D, wide_rows), dim3(unsigned(p.n_blocks * per_block)),
                          dim3(4 * wide_rows), 0, st, p);
     } else {
       hipLaunchKernelGGL(pick(D, kPreBits, tiled ? kPreF16T : kPreF16), dim3(unsigned(grid)),
                          dim3(threads), 0, st, p);
     }
     TQKV_LAUNCHED();
+    if (part_bytes) {
+      merge(p);
+      TQKV_LAUNCHED();
+    }
     return ok();
   }
+  if (part_bytes) use_parts(a, ws);
   hipLaunchKernelGGL(fn, dim3(unsigned(grid)), dim3(threads), 0, st, a);
   TQKV_LAUNCHED();
+  if (part_bytes) {
+    merge(a);
+    TQKV_LAUNCHED();
+  }
   return ok();
 }
 

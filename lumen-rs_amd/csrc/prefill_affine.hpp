@@ -119,10 +119,11 @@ struct Args {
   Seg seg[2];
   int64_t n0, total;  // keys in segment 0; keys in all
   int64_t q_start, k_start, window;
-  // Key splits: split s covers keys [s * split_len, (s + 1) * split_len).
+  // Key splits: split s covers keys split_lo + [s * split_len, (s + 1) * split_len).
   // With part_o set, a row's (o unnormalized, max in log2 units, sum) go to
   // slot split_base + s of n_part, row index (b * L + l) * H + h.
   int n_splits, split_len, split_base, n_part;
+  int64_t split_lo;
   float* part_o;
   float* part_m;
   float* part_l;
@@ -669,7 +670,7 @@ void prefill_affine_kernel(const Args a) {
   const int64_t qa_lo = a.q_start + row0 / a.G, qa_hi = a.q_start + (row_end - 1) / a.G;
 
   // Visible key indices of the block, within its split.
-  int64_t kk_lo = int64_t(split) * a.split_len, kk_hi = a.total - 1;
+  int64_t kk_lo = a.split_lo + int64_t(split) * a.split_len, kk_hi = a.total - 1;
   if (kk_lo + a.split_len - 1 < kk_hi) kk_hi = kk_lo + a.split_len - 1;
   if (a.causal) {
     if (qa_hi - a.k_start < kk_hi) kk_hi = qa_hi - a.k_start;

@@ -75,7 +75,7 @@ void prefill_wide_kernel(const Args a) {
   const int64_t row0 = int64_t(blk) * kRows;
   const int64_t row_end = row0 + kRows < rows ? row0 + kRows : rows;
   const int64_t qa_lo = a.q_start + row0 / a.G, qa_hi = a.q_start + (row_end - 1) / a.G;
-  int64_t kk_lo = int64_t(split) * a.split_len, kk_hi = a.total - 1;
+  int64_t kk_lo = a.split_lo + int64_t(split) * a.split_len, kk_hi = a.total - 1;
   if (kk_lo + a.split_len - 1 < kk_hi) kk_hi = kk_lo + a.split_len - 1;
   if (a.causal) {
     if (qa_hi - a.k_start < kk_hi) kk_hi = qa_hi - a.k_start;

@@ -67,6 +67,27 @@ int32_t scratch_for_current_device(size_t bytes, void** out) {
   return TQKV_OK;
 }
 
+bool scratch_optional(size_t bytes, hipStream_t st, void** out) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  bool grow = true;
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    grow = g_scratch.size() <= size_t(dev) || g_scratch[size_t(dev)].bytes < bytes;
+  }
+  if (grow) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(st, &status);
+    if (e != hipSuccess || status != hipStreamCaptureStatusNone) {
+      if (e != hipSuccess) (void)hipGetLastError();
+      return false;
+    }
+  }
+  if (scratch_for_current_device(bytes, out) == TQKV_OK) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 int32_t scratch_release_all() {
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   int dev = 0;

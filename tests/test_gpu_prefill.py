@@ -246,6 +246,36 @@ def test_prefill_wide_heads_match_in_block(T, monkeypatch, B, H, Hkv, D, L, N, q
         assert np.array_equal(out.numpy(), got["0"]), f"workspace of {ws_bytes} bytes"
 
 
+@pytest.mark.parametrize("B,H,Hkv,D,L,N,q_start,k_start,causal,window", [
+    (1, 8, 4, 64, 33, 1025, 992, 0, True, -1),      # two splits, the last 513 keys
+    (2, 16, 4, 128, 20, 2600, 2580, 0, True, -1),   # five
+    (1, 8, 8, 128, 5, 4096, 0, 0, False, -1),       # eight, unmasked
+    (1, 8, 8, 128, 40, 3000, 2900, 0, True, 1500),  # over the window's keys, rows with blind splits
+    (1, 8, 2, 128, 50, 2000, 10, 40, True, -1),     # rows before any key, 20 keys seen: no split
+    (1, 16, 8, 256, 7, 1700, 1693, 0, True, -1),
+    (1, 32, 2, 512, 9, 1999, 1990, 0, True, -1)])
+def test_prefill_key_splits(T, monkeypatch, B, H, Hkv, D, L, N, q_start, k_start, causal, window):
+    # Short chunks over long contexts split the keys over workgroups and merge
+    # the partials: against the oracle, and the same bits whether the keys are
+    # dequantized once or in every block.
+    print(f"[prefill-splits] B={B} H={H}/{Hkv} D={D} L={L} N={N} window={window}", flush=True)
+    q = kv_bf16((B, H, L, D), D + N)
+    k = kv_bf16((B, Hkv, N, D), D + N + 1, frac=0.01, mult=10.0)
+    v = kv_bf16((B, Hkv, N, D), D + N + 2, frac=0.01, mult=10.0)
+    (kh, kd), (vh, vd) = _cache(k, 64, 4, N + 5), _cache(v, 64, 4, N + 5)
+    got = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("TQKV_PREFILL_DEQUANT_ONCE", mode)
+        got[mode] = run(T, q, [(kd, vd, N + 5, N, False)], B, H, Hkv, L, D, 64, 4, 4, D ** -0.5,
+                        q_start, k_start, causal, window)
+    assert np.array_equal(got["0"], got["1"])
+    want = want_mlx(q, kh, vh, 64, 4, 4, D ** -0.5, causal=causal, q_start=q_start,
+                    first_held=k_start, window=window)
+    check(got["1"], want, "splits")
+    if causal and k_start > q_start:
+        assert np.all(got["1"][:, :, :k_start - q_start] == 0)
+
+
 @pytest.mark.parametrize("case", [0, 1, 3, 4, 5, 7, 9, 10, 12, 13])
 def test_prefill_dequantize_once_is_bit_identical(T, monkeypatch, case):
     # Keys dequantized once into scratch (mlx::dequantize's bits) and then
