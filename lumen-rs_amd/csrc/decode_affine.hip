@@ -14,6 +14,7 @@ int32_t shared_prefix_partials(const uint16_t* q, int B, int H, int H_kv, int D,
 int shared_prefix_block_rows(int D);
 bool tile_decode_supported(int D, int bk, int bv);
 int tile_decode_rows();
+bool tile_decode_wide(int bk, int bv);
 int32_t tile_decode(const uint16_t* q, int B, int H, int H_kv, int D, int gs, int bk, int bv,
                     float scale, const tqkv_affine_seg* segs, int n_segs, int n_splits,
                     int split_len, int n_part, float* part_o, float* part_m, float* part_l,
@@ -296,9 +297,9 @@ int group_heads(int D, int bk, int bv, int G, int gs, int64_t max_rows = 0) {
   return 0;
 }
 
-// Head dim 512 decodes through the tile kernel (the prefill kernel's f16
-// variant, a sequence's heads as the rows of a block): its scores and
-// values run on the matrix cores, where the dot2 kernel spends a 64-lane
+// Head dim 512 decodes through the tile kernels (decode_wide_kernel at 4 and
+// 8 bits, else the prefill kernel's f16 variant, a sequence's heads as the
+// rows of a block): their scores and values run on the matrix cores, where the dot2 kernel spends a 64-lane
 // reduction per token and head at that width (measured 3-9x slower). No
 // fused append there (that needs the MFMA decode kernel), and
 // TQKV_DECODE_KERNEL=dot2 keeps the dot2 kernel.
@@ -368,7 +369,7 @@ struct AppendDst {
 // How a decode call splits its keys, and the workspace bytes that needs (0:
 // none). Only the segments' lengths and shared flags matter.
 struct DecodePlan {
-  bool tile = false;  // the tile kernel (use_tile), splits as below
+  bool tile = false;  // the tile kernels (use_tile), splits as below
   bool shared_path = false;
   // Shared prefix read once: prefix splits, then the suffix's.
   int sp_p = 0, split_len_p = 0, sp_s = 0;
@@ -381,10 +382,11 @@ struct DecodePlan {
 };
 
 // Gk: the query heads one decode launch serves (kernel_heads).
-// waves: the launch's wavefronts a workgroup (decode_waves); tile: the
-// tile kernel decodes (use_tile).
+// waves: the launch's wavefronts a workgroup (decode_waves); tile_keys: the
+// least keys a split where a tile kernel decodes (use_tile), 0 otherwise.
+constexpr int kTileKeys = 256;
 DecodePlan plan_decode(int B, int H, int H_kv, int D, int Gk, int waves,
-                       const tqkv_affine_seg* segs, int n_segs, bool app, bool tile = false) {
+                       const tqkv_affine_seg* segs, int n_segs, bool app, int tile_keys = 0) {
   DecodePlan pl;
   const int G = H / H_kv;
   const int64_t total = segs[0].n + (n_segs == 2 ? segs[1].n : 0);
@@ -410,17 +412,18 @@ DecodePlan plan_decode(int B, int H, int H_kv, int D, int Gk, int waves,
     pl.need = size_t(B) * H * pl.n_part * row * sizeof(float);
     return pl;
   }
-  if (tile) {
+  if (tile_keys) {
     // About 256 workgroups (one a CU: the tile kernel's LDS holds one),
-    // never under 256 keys a split.
+    // never under tile_keys keys a split.
     const int rows = prefill::tile_decode_rows();
     const int64_t units = int64_t(B) * H_kv * ((G + rows - 1) / rows);
     int64_t want = (256 + units - 1) / units;
-    const int64_t most = (total + 255) / 256;
+    const int64_t most = (total + tile_keys - 1) / tile_keys;
     if (want > most) want = most;
     if (want < 1) want = 1;
     int64_t len = (total + want - 1) / want;
-    len = (len + 63) / 64 * 64;
+    const int unit = tile_keys < kTileKeys ? tile_keys : 64;  // the wide kernel's tiles, or 64
+    len = (len + unit - 1) / unit * unit;
     pl.tile = true;
     pl.split_len = len;
     pl.n_splits = int((total + len - 1) / len);
@@ -509,16 +512,27 @@ int32_t decode_affine(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, int
 
   const int waves = decode_waves(D, bits_k, bits_v, Gk, group_size, mfma);
   a.out = out;
-  const DecodePlan pl = plan_decode(B, H, H_kv, D, Gk, waves, segs, n_segs, app != nullptr, tile);
+  DecodePlan pl = plan_decode(B, H, H_kv, D, Gk, waves, segs, n_segs, app != nullptr,
+                              tile ? kTileKeys : 0);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   void* ws = workspace;
+  if (tile && pl.need > 0 && prefill::tile_decode_wide(bits_k, bits_v)) {
+    // The wide kernel's splits go down to one of its tiles where that puts
+    // more of the chip to work (with 256 workgroups both plans are the same):
+    // B = 2, 4 KV heads, 700 keys 24.6 us at 256 keys a split, 18.8 at 128.
+    // Only with room for the partials, so that no call needs more workspace
+    // than the 256-key plan does (and none for a context of one split).
+    const DecodePlan fine = plan_decode(B, H, H_kv, D, Gk, waves, segs, n_segs, false,
+                                        kTileKeys / 2);
+    if (ws ? workspace_bytes >= fine.need : scratch_optional(fine.need, st, &ws)) pl = fine;
+  }
   if (pl.need > 0) {
     if (!ws) {
       if (int32_t rc = scratch_for_current_device(pl.need, &ws)) return rc;
-    } else if (workspace_bytes < pl.need) {
+    } else if (workspace && workspace_bytes < pl.need) {
       return fail(TQKV_EINVAL_ARG, "workspace of %zu bytes, need %zu", workspace_bytes, pl.need);
     }
   }
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
 
   if (pl.tile) {
     float* po = static_cast<float*>(ws);
@@ -634,7 +648,7 @@ size_t decode_need_bytes(int B, int H, int H_kv, int D, int group_size, int bits
   KernelFn fn = Gp ? pick(D, bits_k, bits_v, Gp, group_size, max_rows) : nullptr;
   const bool mfma = fn && fn == pick_mfma_only(D, bits_k, bits_v, Gp, group_size);
   return plan_decode(B, H, H_kv, D, Gk, decode_waves(D, bits_k, bits_v, Gk, group_size, mfma),
-                     segs, n_segs, app, tile).need;
+                     segs, n_segs, app, tile ? kTileKeys : 0).need;
 }
 }  // namespace tqkv
 

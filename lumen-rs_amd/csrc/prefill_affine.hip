@@ -246,8 +246,11 @@ namespace prefill {
 // (rows (b, g) of a KV head), the prefix's keys are split over the grid,
 // and each split's (o, m, l) go to slots [0, n_splits) of the decode's
 // partials [B, H, n_part]. Rows b * H + h line up with the decode kernel's.
-bool tile_decode_supported(int D, int bk, int bv) { return D == 512 && pick(D, bk, bv, true); }
+bool tile_decode_supported(int D, int bk, int bv) {
+  return D == 512 && (pick_decode_wide(bk, bv) || pick(D, bk, bv, true));
+}
 int tile_decode_rows() { return Shape<512, true>::kRows; }
+bool tile_decode_wide(int bk, int bv) { return pick_decode_wide(bk, bv) != nullptr; }
 
 // Decode through the tile kernel (f16 operands): each sequence's G query
 // heads of a KV head are the rows of one block (one position, L = 1), the
@@ -259,7 +262,7 @@ int32_t tile_decode(const uint16_t* q, int B, int H, int H_kv, int D, int gs, in
                     float scale, const tqkv_affine_seg* segs, int n_segs, int n_splits,
                     int split_len, int n_part, float* part_o, float* part_m, float* part_l,
                     uint16_t* out, hipStream_t st) {
-  KernelFn fn = pick(D, bk, bv, true);
+  const KernelFn wide = pick_decode_wide(bk, bv), fn = wide ? wide : pick(D, bk, bv, true);
   if (!fn || D != 512) return fail(TQKV_EUNSUPPORTED, "tile decode D=%d bits %d/%d", D, bk, bv);
   Args a{};
   a.q = q;
@@ -300,7 +303,8 @@ int32_t tile_decode(const uint16_t* q, int B, int H, int H_kv, int D, int gs, in
   a.n_blocks = int(blocks);
   const int64_t grid = blocks * n_splits * H_kv * int64_t(B);
   if (grid > 0x7fffffff) return fail(TQKV_EINVAL_SHAPE, "grid too large");
-  hipLaunchKernelGGL(fn, dim3(unsigned(grid)), dim3(S::kThreads), 0, st, a);
+  static_assert(S::kRows == 16, "16 heads a block in both kernels");
+  hipLaunchKernelGGL(fn, dim3(unsigned(grid)), dim3(wide ? 512 : S::kThreads), 0, st, a);
   TQKV_LAUNCHED();
   return TQKV_OK;
 }

@@ -1332,15 +1332,29 @@ KernelFn pick_d512(int bk, int bv, bool h16);
 // row.
 KernelFn pick_wide(int D, int rows);
 
+// The kernel of decode_wide.hip for head dim 512 (4- and 8-bit widths, null
+// otherwise), 512 threads, 16 heads a block.
+KernelFn pick_decode_wide(int bk, int bv);
+
 template <int D, int BK, bool H16>
 KernelFn pick_bv(int bv) {
-  switch (bv) {
-    case 2: return prefill_affine_kernel<D, BK, 2, H16>;
-    case 3: return prefill_affine_kernel<D, BK, 3, H16>;
-    case 4: return prefill_affine_kernel<D, BK, 4, H16>;
-    case 5: return prefill_affine_kernel<D, BK, 5, H16>;
-    case 6: return prefill_affine_kernel<D, BK, 6, H16>;
-    case 8: return prefill_affine_kernel<D, BK, 8, H16>;
+  // Decode at head dim 512 over 4- and 8-bit widths is decode_wide_kernel's.
+  if constexpr (D == 512 && H16 && (BK == 4 || BK == 8)) {
+    switch (bv) {
+      case 2: return prefill_affine_kernel<D, BK, 2, H16>;
+      case 3: return prefill_affine_kernel<D, BK, 3, H16>;
+      case 5: return prefill_affine_kernel<D, BK, 5, H16>;
+      case 6: return prefill_affine_kernel<D, BK, 6, H16>;
+    }
+  } else {
+    switch (bv) {
+      case 2: return prefill_affine_kernel<D, BK, 2, H16>;
+      case 3: return prefill_affine_kernel<D, BK, 3, H16>;
+      case 4: return prefill_affine_kernel<D, BK, 4, H16>;
+      case 5: return prefill_affine_kernel<D, BK, 5, H16>;
+      case 6: return prefill_affine_kernel<D, BK, 6, H16>;
+      case 8: return prefill_affine_kernel<D, BK, 8, H16>;
+    }
   }
   return nullptr;
 }

@@ -1,5 +1,5 @@
-// Instantiations of the affine prefill kernel for head dim 512 (bf16
-// operands only: the f16 variant serves shared-prefix decode up to D = 256).
+// Instantiations of the affine prefill kernel for head dim 512 (the f16
+// variant decodes the widths that decode_wide_kernel does not take).
 #include "prefill_affine.hpp"
 
 namespace tqkv {

@@ -416,6 +416,37 @@ def test_decode_two_segments(T, kernel, B, H, Hkv, D, n1, n2, shared, bk, bv):
     check_close(got, wf, wm)
 
 
+@pytest.mark.parametrize("B,H,Hkv,n1,n2,gs,bk,bv", [
+    (1, 2, 2, 1, 0, 32, 4, 4),        # one key, one head a block
+    (2, 16, 1, 127, 0, 64, 8, 8),     # one short of a 128-key tile
+    (1, 32, 2, 128, 0, 128, 4, 8),    # a whole tile
+    (1, 32, 1, 257, 0, 64, 8, 4),     # a second tile of one key; two blocks of 16 heads
+    (1, 17, 1, 300, 0, 32, 8, 8),     # a last block of one head
+    (1, 8, 2, 130, 127, 64, 4, 4),    # the segments' seam inside a tile, three splits of 128
+    (1, 24, 2, 3, 140, 32, 8, 4),     # and near a tile's start
+    (40, 16, 8, 200, 33, 64, 4, 4),   # one split a unit (320 units): whole and partial tiles
+])
+def test_decode_head_dim_512_tiles(T, B, H, Hkv, n1, n2, gs, bk, bv):
+    """Head dim 512 at the edges of its 128-key tiles, 16-head blocks, splits
+    and segments: the oracle over the segments' concatenation."""
+    print(f"[decode-512] B={B} H={H}/{Hkv} n={n1}+{n2} gs={gs} bits={bk}/{bv}", flush=True)
+    assert T.decode_kernel_name(H, Hkv, 512, gs, bk, bv) == "tiles"
+    D = 512
+    q = kv_bf16((B, H, 1, D), 71 + n1, std=D ** -0.5 * 4)
+    ks, vs, segs = [], [], []
+    for i, n in enumerate((n1, n2)):
+        if n:
+            k, v = kv_bf16((B, Hkv, n, D), 72 + 2 * i), kv_bf16((B, Hkv, n, D), 73 + 2 * i)
+            (kh, kd), (vh, vd) = _cache(k, gs, bk, n + 5), _cache(v, gs, bv, n + 5)
+            ks.append(kh), vs.append(vh), segs.append((kd, vd, n + 5, n, False))
+    got = run_decode(T, q, segs, B, H, Hkv, D, gs, bk, bv, 1.0)
+    kfull = tuple(np.concatenate(a, axis=2) for a in zip(*ks))
+    vfull = tuple(np.concatenate(a, axis=2) for a in zip(*vs))
+    wf, _, _ = O.attend_affine(q, kfull, vfull, gs, bk, bv, 1.0)
+    wm, _, _ = O.attend_affine(q, kfull, vfull, gs, bk, bv, 1.0, dequant="bf16")
+    check_close(got, wf, wm)
+
+
 def test_decode_shared_prefix_plus_suffix(T, kernel):
     # sdpa_split semantics (native_attention.rs:174-208): one softmax over a
     # shared batch-1 prefix and each row's own suffix.
