@@ -1115,7 +1115,7 @@ def codebook_main(T, hip, args):
                      "codebook cache: 3-bit Lloyd-Max codes (u8) + f32 sigma, K and V rotated",
          "batch": B, "q_heads": H, "kv_heads": HKV, "head_dim": D, "context": N,
          "bits_k": BITS, "bits_v": BITS},
-        _hbm(alg / (ms * 1e-3) / 1e9, "one call: cb_rotate_q_kernel + cb_decode_kernel<256,2,false> + cb_merge_kernel", alg, ms),
+        _hbm(alg / (ms * 1e-3) / 1e9, "one call: cb_matmul_kernel (q R) + cb_decode_kernel<256> + cb_merge_kernel + cb_matmul_kernel (o R^T)", alg, ms),
         {"workspace_bytes": wsb}, settle, steps)
     print(json.dumps(result))
 

@@ -18,10 +18,10 @@
 // they stay in flight over the work between takes `loaded` and `moved` below
 // (without: 29.8 us at the shape above, with: 28.0).
 //
-// Measured, the tile kernel -> this one, a call with its merge: the shape above
-// 36.9 -> 28.0 us, with 8-bit codes 43.2 -> 31.2; B = 16, 16,000 keys 174 ->
-// 97; one sequence of 120,000 keys (8 bits) 131 -> 76, of 256 keys 27.0 ->
-// 22.4, of 20 keys 14.2 -> 13.6.
+// Measured, the tile kernel -> this one, a step (append, decode, merge): the
+// shape above 36.9 -> 28.0 us, with 8-bit codes 43.2 -> 31.2; B = 16, 16,000
+// keys 174 -> 97; one sequence of 120,000 keys (8 bits) 131 -> 74, of 257 keys
+// 27.0 -> 16.4 (three splits of 128), of 21 keys 14.2 -> 13.5.
 #include "prefill_affine.hpp"
 
 namespace tqkv {
