@@ -390,8 +390,8 @@ int32_t tqkv_decode_attend_codebook_qjl(const uint16_t* q, int32_t B, int32_t H,
  * q: bf16 [B, H, L, D]; out: bf16 [B, H, L, D]; segs as for
  * tqkv_decode_attend_affine (1 or 2: a shared prefix, then a suffix).
  * D in {64, 128, 256, 512}; bits_k, bits_v in {2, 3, 4, 5, 6, 8}; group_size in
- * {32, 64, 128}. Uses the library's scratch for the dequantize-once rows:
- * calls that use it (this one, and decodes given a null workspace) must not
+ * {32, 64, 128}. Uses the library's scratch for the dequantize-once rows and
+ * the split partials: calls that use it (this one, and decodes given a null workspace) must not
  * overlap in time on one device; tqkv_prefill_attend_affine_ws takes a
  * workspace instead.
  */
@@ -608,7 +608,7 @@ int32_t tqkv_cache_append_decode(tqkv_cache* cache, const uint16_t* k, const uin
  * bf16(centroid * sigma) (lloyd_max_dequantize_scaled), keys with QJL signs
  * corrected to K_eff, queries rotated by R and the output rotated back (the
  * cache holds rotated rows); this uses library scratch. bf16 caches attend
- * their rows as they are. An attached prefix is read for affine caches only.
+ * their rows as they are, without library scratch. An attached prefix is read for affine caches only.
  * q: bf16 [B, H, L, D]; out: bf16 [B, H, L, D].
  */
 int32_t tqkv_cache_prefill_attend(const tqkv_cache* cache, const uint16_t* q, int32_t H,

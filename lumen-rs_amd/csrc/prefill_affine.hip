@@ -6,10 +6,13 @@
 #include <cstring>
 
 #include "prefill_affine.hpp"
+#include "prefill_plan.hpp"
 
 namespace tqkv {
 namespace prefill {
 namespace {
+
+static_assert(kTile == prefillplan::kTileKeys, "whole tiles a split");
 
 bool valid_bits(int bits) {
   return bits == 2 || bits == 3 || bits == 4 || bits == 5 || bits == 6 || bits == 8;
@@ -193,16 +196,6 @@ int64_t once_blocks(int D, int64_t total) {
 // The scratch that path may take (bf16 K and V of every visible key); larger
 // contexts dequantize in every block instead.
 constexpr size_t kOnceMaxBytes = size_t(4) << 30;
-
-// Key splits of a chunk whose row blocks would leave CUs idle (a short chunk
-// over a long context): workgroups wanted, keys a split holds at least (a
-// split pays its partials' write and read), bytes of partials at most.
-// Measured (4-bit, without and with): 16 / 8 heads, D = 128, 64 rows over
-// 24,000 keys 569 and 42 us, 147 rows over 16,384 565 and 55; D = 256, 256
-// rows over 16,384 661 and 104; 32 / 2 heads, D = 512, 64 rows over 20,000
-// 2,700 and 134 (with the wide kernel).
-constexpr int64_t kSplitWorkgroups = 256, kSplitMinKeys = 512;
-constexpr size_t kSplitMaxBytes = size_t(1) << 30;
 
 // The splits' partials of each row (slots (row, split), row = (b L + l) H +
 // h) combined and written as bf16: four channels a thread.
@@ -437,10 +430,7 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   a.q_start = q_start;
   a.k_start = k_start;
   a.window = window < 0 ? -1 : window;
-  a.n_splits = 1;
-  a.split_len = int(a.total + kTile - 1) / kTile * kTile;
   a.split_base = 0;
-  a.n_part = 1;
 
   int rows_per_block = 0, threads = 0;
   switch (D) {
@@ -451,31 +441,17 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   }
   const int64_t blocks = (int64_t(L) * a.G + rows_per_block - 1) / rows_per_block;
   if (blocks * H_kv * B > 0x7fffffff) return fail(TQKV_EINVAL_SHAPE, "grid too large");
-  // Key splits, over the keys some row can see, with the library's scratch
-  // (a caller's workspace holds the dequantized rows only).
   const int64_t units = blocks * H_kv * B, q_rows = int64_t(B) * H * L;
-  if (library_scratch && units * 2 <= kSplitWorkgroups) {
-    int64_t lo = 0, hi = a.total - 1;
-    if (a.causal) {
-      if (q_start + L - 1 - k_start < hi) hi = q_start + L - 1 - k_start;
-      if (a.window >= 0 && q_start - a.window + 1 - k_start > lo) lo = q_start - a.window + 1 - k_start;
-    }
-    lo = lo / kTile * kTile;
-    int64_t splits = kSplitWorkgroups / units;
-    if (splits > (hi - lo) / kSplitMinKeys) splits = (hi - lo) / kSplitMinKeys;
-    if (splits >= 2 && size_t(q_rows) * size_t(splits) * (D + 2) * sizeof(float) <= kSplitMaxBytes) {
-      a.split_len = int((hi + 1 - lo + splits * kTile - 1) / (splits * kTile) * kTile);
-      a.n_splits = a.n_part = int((hi + 1 - lo + a.split_len - 1) / a.split_len);
-      a.split_lo = lo;
-    }
-  }
-  size_t part_bytes = a.n_splits > 1 ? size_t(q_rows) * a.n_splits * (D + 2) * sizeof(float) : 0;
-  const auto no_splits = [&] {
-    a.n_splits = a.n_part = 1;
-    a.split_len = int(a.total + kTile - 1) / kTile * kTile;
-    a.split_lo = 0;
-    part_bytes = 0;
+  const prefillplan::Chunk chunk{B, H, H_kv, L, D, a.total, q_start, k_start, a.causal != 0,
+                                 a.window, blocks, bf16_rows, library_scratch};
+  size_t part_bytes = 0;
+  const auto use_splits = [&](const prefillplan::Splits& sp) {
+    a.n_splits = a.n_part = int(sp.n);
+    a.split_len = int(sp.len);
+    a.split_lo = sp.lo;
+    part_bytes = sp.bytes;
   };
+  use_splits(prefillplan::key_splits(chunk));
   a.n_blocks = int(blocks);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // The partials at p (16-byte aligned), and the merge after the kernel.
@@ -513,7 +489,7 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   if (library_scratch && (once || part_bytes)) {
     const size_t rows_bytes = once ? need : 0;
     bool held = part_bytes && scratch_optional(rows_bytes + part_bytes, st, &ws);
-    if (!held) no_splits();
+    if (!held) use_splits(prefillplan::no_splits(chunk));
     if (once && !held) {
       if (blocks >= kOnceBlocks || once_env) {
         if (int32_t rc = scratch_for_current_device(need, &ws)) return rc;

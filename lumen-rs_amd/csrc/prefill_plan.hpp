@@ -1,0 +1,80 @@
+// How a prefill call splits its work and what scratch that takes, as plain
+// C++ (no HIP): prefill_affine.hip launches by it, the tests check it on the
+// CPU over all forms of a call.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+namespace tqkv {
+namespace prefillplan {
+
+constexpr int64_t kTileKeys = 64;  // keys a step of every prefill kernel
+
+struct Chunk {
+  int64_t B, H, H_kv, L, D;
+  int64_t total;  // keys of both segments
+  int64_t q_start, k_start;
+  bool causal;
+  int64_t window;        // < 0: none
+  int64_t blocks;        // row blocks a KV head in the in-block kernel
+  bool bf16_rows;        // K and V are bf16 rows, not packed codes
+  bool library_scratch;  // else a caller's workspace, which holds rows only
+};
+
+// The keys [lo, hi] that some row of the chunk sees, lo down to a whole tile;
+// hi < lo where no row sees any.
+struct Visible {
+  int64_t lo, hi;
+};
+inline Visible visible_keys(const Chunk& c) {
+  int64_t lo = 0, hi = c.total - 1;
+  if (c.causal) {
+    if (c.q_start + c.L - 1 - c.k_start < hi) hi = c.q_start + c.L - 1 - c.k_start;
+    if (c.window >= 0 && c.q_start - c.window + 1 - c.k_start > lo)
+      lo = c.q_start - c.window + 1 - c.k_start;
+  }
+  return Visible{lo / kTileKeys * kTileKeys, hi};
+}
+
+// Key splits of a chunk whose row blocks would leave CUs idle (a short chunk
+// over a long context): workgroups wanted, keys a split holds at least (a
+// split pays its partials' write and read), bytes of partials at most.
+// Measured (4-bit, without and with): 16 / 8 heads, D = 128, 64 rows over
+// 24,000 keys 569 and 42 us, 147 rows over 16,384 565 and 55; D = 256, 256
+// rows over 16,384 661 and 104; 32 / 2 heads, D = 512, 64 rows over 20,000
+// 2,700 and 134 (with the wide kernel).
+// Not over bf16 rows: a codebook cache's dequantized rows and rotated queries
+// sit in the library scratch that the partials would take, and a bf16 cache's
+// chunk uses no scratch, so that caches on different streams stay independent.
+constexpr int64_t kSplitWorkgroups = 256, kSplitMinKeys = 512;
+constexpr size_t kSplitMaxBytes = size_t(1) << 30;
+
+struct Splits {
+  int64_t n = 1, len = 0, lo = 0;  // split s: keys lo + [s * len, (s + 1) * len)
+  size_t bytes = 0;                // of partials (0: the keys are not split)
+};
+inline Splits no_splits(const Chunk& c) {
+  Splits s;
+  s.len = (c.total + kTileKeys - 1) / kTileKeys * kTileKeys;
+  return s;
+}
+inline Splits key_splits(const Chunk& c) {
+  Splits s = no_splits(c);
+  const int64_t units = c.blocks * c.H_kv * c.B, rows = c.B * c.H * c.L;
+  if (c.bf16_rows || !c.library_scratch || units * 2 > kSplitWorkgroups) return s;
+  const Visible v = visible_keys(c);
+  int64_t n = kSplitWorkgroups / units;
+  if (n > (v.hi - v.lo) / kSplitMinKeys) n = (v.hi - v.lo) / kSplitMinKeys;
+  const size_t slot = size_t(c.D + 2) * sizeof(float);
+  if (n < 2 || size_t(rows) * size_t(n) * slot > kSplitMaxBytes) return s;
+  const int64_t keys = v.hi + 1 - v.lo;
+  s.len = (keys + n * kTileKeys - 1) / (n * kTileKeys) * kTileKeys;
+  s.n = (keys + s.len - 1) / s.len;
+  s.lo = v.lo;
+  s.bytes = s.n > 1 ? size_t(rows) * size_t(s.n) * slot : 0;
+  return s;
+}
+
+}  // namespace prefillplan
+}  // namespace tqkv

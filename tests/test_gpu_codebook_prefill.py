@@ -129,6 +129,75 @@ def test_bf16_cache_prefill(T):
         check(out.numpy(), want, f"bf16 chunk {i}")
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,N,L,bits,qjl_words", [
+    (128, 16, 8, 4096, 256, 4, 0), (128, 16, 8, 8192, 200, 3, 0), (128, 8, 4, 2100, 20, 4, 2),
+    (256, 8, 4, 4096, 64, 4, 0), (512, 32, 2, 2100, 24, 4, 0), (64, 8, 8, 2600, 30, 4, 4)])
+def test_codebook_cache_prefill_of_a_short_chunk_over_a_long_context(T, D, Hq, Hkv, N, L, bits,
+                                                                     qjl_words):
+    # The chunk's rotated queries and dequantized rows live in the library
+    # scratch while it runs. Three times over, the scratch grown by the first:
+    # the same bits each time, and the oracle's result.
+    B = 1
+    c = T.Cache(T.CACHE_CODEBOOK, B, Hkv, D, D, bits_k=bits, bits_v=bits, qjl_words=qjl_words,
+                max_size=N, keep=0, seed=42, encode=1)
+    k = kv_bf16((B, Hkv, N, D), 80 + D, frac=0.02, mult=8.0)
+    v = kv_bf16((B, Hkv, N, D), 90 + D, frac=0.02, mult=8.0)
+    q = kv_bf16((B, Hq, L, D), 100 + D)
+    dk, dv, dq = T.DeviceArray.of(k), T.DeviceArray.of(v), T.DeviceArray.of(q)
+    view = c.append(dk.ptr, dv.ptr, N)
+    assert view.n == N
+    T.hip().sync()
+    T.scratch_release()
+    got = []
+    for i in range(3):
+        out = T.DeviceArray((B, Hq, L, D), np.uint16, np.full((B, Hq, L, D), 0x7FC0, np.uint16))
+        print(f"[cb-prefill] long D={D} {Hq}/{Hkv} N={N} L={L} qjl={qjl_words} pass {i}", flush=True)
+        c.prefill_attend(dq.ptr, Hq, L, D ** -0.5, out.ptr)
+        T.hip().sync()
+        got.append(out.numpy())
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    bufs = c.buffers()
+    R = T.rotation_matrix(D, 42).astype(np.float64).T  # R_eff of the GPU cache's encode
+    _, cent = T.lloyd_max(bits)
+    cent = cent.astype(np.float32)
+    vi = 4 if qjl_words else 2
+    kc, vc = (T.view_slot(bufs, i, B * Hkv, np.uint8, D)[:, :N] for i in (0, vi))
+    ks, vs = (T.view_slot(bufs, i, B * Hkv, np.float32, 1)[:, :N, 0] for i in (1, vi + 1))
+    K = dequant(cent, kc, ks).reshape(-1, D)
+    if qjl_words:
+        m = 32 * qjl_words
+        sg = T.view_slot(bufs, 2, B * Hkv, np.uint32, qjl_words)[:, :N].reshape(-1, qjl_words)
+        rn = T.view_slot(bufs, 3, B * Hkv, np.float32, 1)[:, :N, 0].reshape(-1)
+        K = O.qjl_apply_correction(K, sg, rn, T.qjl_matrix(D, m, 43)[:m], m)
+    K = K.reshape(B, Hkv, N, D)
+    V = dequant(cent, vc, vs).reshape(B, Hkv, N, D)
+    V = O.bf16_from_f32((O.bf16_to_f32(V).astype(np.float64) @ R).astype(np.float32))
+    qr = O.bf16_from_f32((O.bf16_to_f32(q).astype(np.float64) @ R.T).astype(np.float32))
+    want, _, _ = O.attend_bf16(qr, K, V, D ** -0.5, causal=True, q_start=N - L, first_held=0)
+    check(got[0], want, f"long D={D}")
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,N,L", [(128, 16, 4, 3000, 20), (256, 8, 2, 2500, 40),
+                                          (512, 16, 2, 2100, 9)])
+def test_bf16_cache_prefill_uses_no_library_scratch(T, D, Hq, Hkv, N, L):
+    # A short chunk over a long context: caches on different streams share
+    # nothing, so the call must leave the library's scratch alone.
+    B = 1
+    c = T.Cache(T.CACHE_BF16, B, Hkv, D, D)
+    k, v, q = (kv_bf16(s, 40 + i) for i, s in enumerate(((B, Hkv, N, D),) * 2 + ((B, Hq, L, D),)))
+    dk, dv, dq = T.DeviceArray.of(k), T.DeviceArray.of(v), T.DeviceArray.of(q)
+    c.append(dk.ptr, dv.ptr, N)
+    out = T.DeviceArray((B, Hq, L, D), np.uint16)
+    T.hip().sync()
+    T.scratch_release()
+    print(f"[cb-prefill] bf16 D={D} N={N} L={L}", flush=True)
+    c.prefill_attend(dq.ptr, Hq, L, D ** -0.5, out.ptr)
+    T.hip().sync()
+    assert T.scratch_bytes() == 0
+    want, _, _ = O.attend_bf16(q, k, v, D ** -0.5, causal=True, q_start=N - L, first_held=0)
+    check(out.numpy(), want, f"bf16 long D={D}")
+
+
 def test_compress_one_qjl_prefill_is_unsupported(T):
     # compress_one's QJL signs are of the original-basis residual; the
     # reference prefills with QJL only over its GPU cache's rotated-residual

@@ -1,0 +1,103 @@
+"""The prefill's plan (lumen-rs_amd/csrc/prefill_plan.hpp) over all forms of a
+call, on the CPU: which keys a chunk sees, and how they are split."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+BUILD = os.path.join(ROOT, "tests", "_build")
+LIB = os.path.join(BUILD, "libprefillplanhost.so")
+FIELDS = ("B", "H", "Hkv", "L", "D", "total", "q_start", "k_start", "causal", "window", "blocks",
+          "bf16_rows", "library_scratch")
+ROWS = {64: 128, 128: 256, 256: 128, 512: 64}  # rows a block of the in-block kernel
+
+
+@pytest.fixture(scope="module")
+def host():
+    os.makedirs(BUILD, exist_ok=True)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC",
+                    "-I", os.path.join(ROOT, "lumen-rs_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "prefill_plan_host.cpp"), "-o", LIB], check=True)
+    return ctypes.CDLL(LIB)
+
+
+def ask(fn, c, n):
+    out = (ctypes.c_int64 * n)()
+    fn((ctypes.c_int64 * len(FIELDS))(*(int(c[f]) for f in FIELDS)), out)
+    return list(out)
+
+
+def chunk(rng, **fixed):
+    D = rng.choice((64, 128, 256, 512))
+    Hkv = rng.choice((1, 2, 4, 8))
+    G = rng.choice((1, 2, 3, 4, 8, 16))
+    L = int(2 ** rng.uniform(0, 12))
+    total = int(2 ** rng.uniform(0, 17))
+    c = dict(B=rng.choice((1, 1, 2, 5)), H=Hkv * G, Hkv=Hkv, L=L, D=D, total=total,
+             k_start=rng.choice((0, 0, 40, 100000)), causal=rng.random() < 0.8,
+             window=rng.choice((-1, -1, 1, 100, 1500, 1 << 40)), bf16_rows=False,
+             library_scratch=rng.random() < 0.8)
+    c["q_start"] = rng.choice((c["k_start"] + total - L, 0, c["k_start"] + total // 2))
+    c.update(fixed)
+    c["blocks"] = -(-c["L"] * (c["H"] // c["Hkv"]) // ROWS[c["D"]])
+    return c
+
+
+def seen(c):
+    """The keys that some row sees, by the mask's own rule."""
+    if not c["causal"]:
+        return 0, c["total"] - 1
+    first = max(c["q_start"] - c["k_start"], 0)  # the rows that see a key
+    last = c["q_start"] + c["L"] - 1 - c["k_start"]
+    if c["window"] >= 0:
+        last = min(last, c["total"] + c["window"] - 2)
+    if first > last:
+        return 0, -1
+    return max(0, first - c["window"] + 1) if c["window"] >= 0 else 0, min(c["total"] - 1, last)
+
+
+def test_visible_keys_cover_what_rows_see(host):
+    rng = random.Random(1)
+    for _ in range(3000):
+        c = chunk(rng)
+        lo, hi = ask(host.planhost_visible, c, 2)
+        a, b = seen(c)
+        if a <= b:
+            assert lo % 64 == 0 and lo <= a and hi >= b and hi < c["total"], (c, lo, hi)
+
+
+def test_splits_cover_the_visible_keys(host):
+    rng = random.Random(2)
+    split = 0
+    for _ in range(3000):
+        c = chunk(rng)
+        n, ln, lo, size = ask(host.planhost_splits, c, 4)
+        a, b = seen(c)
+        assert n >= 1 and ln % 64 == 0 and lo % 64 == 0
+        if a <= b:
+            assert lo <= a and lo + n * ln > b, (c, n, ln, lo)
+        assert (size > 0) == (n > 1)
+        if n > 1:
+            split += 1
+            assert c["library_scratch"] and lo + (n - 1) * ln <= b, c  # none is empty
+            assert n * c["blocks"] * c["Hkv"] * c["B"] <= 256
+            assert size == c["B"] * c["H"] * c["L"] * n * (c["D"] + 2) * 4 <= 1 << 30
+    assert split > 100
+
+
+def test_bf16_rows_are_never_split(host):
+    # A codebook cache's chunk attends dequantized rows and rotated queries
+    # that sit in the library scratch, where partials would overwrite them; a
+    # bf16 cache's uses no scratch, so that two caches on two streams do not
+    # meet there.
+    rng = random.Random(3)
+    c = chunk(rng, B=1, H=32, Hkv=8, L=64, D=128, total=8192, q_start=8128, k_start=0, causal=True,
+              window=-1, library_scratch=True)
+    assert ask(host.planhost_splits, c, 4)[0] > 1  # packed codes at this shape are
+    for D in (64, 128, 256, 512):
+        for _ in range(500):
+            n, _, lo, size = ask(host.planhost_splits, chunk(rng, D=D, bf16_rows=True), 4)
+            assert (n, lo, size) == (1, 0, 0)
