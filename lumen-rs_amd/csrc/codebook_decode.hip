@@ -349,9 +349,14 @@ void cb_decode_kernel(const Args a) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) o[j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
   // The weights' exponentials p are held times 2^sv_exp, which puts p * sigma
-  // below 2^15 for sigma < sv_lim; l sums them so scaled.
-  int sv_exp = 0;
-  float sv_lim = 0.0f;
+  // below 2^15 for sigma < sv_lim; l sums them so scaled. The scale follows
+  // the tiles' largest sigmas, down as they pass sv_lim and up as a whole tile
+  // stays below sv_low, so that a weight keeps its 22 bits after a tile of
+  // zeros or of far larger sigmas. (In one tile with sigmas 2^15 times larger
+  // its last bits are below theirs.) Up it stays within 2^64 of the lowest
+  // scale so far, where the older sums (below 2^61) cannot overflow.
+  int sv_exp = 0, sv_top = 90;
+  float sv_lim = 0.0f, sv_low = 0.0f;
 
   int buf = 0;
   for (int64_t base = t0; base < t1; base += T, buf ^= 1) {
@@ -449,13 +454,19 @@ void cb_decode_kernel(const Args a) {
     const float mn = fmaxf(m, mx);
     float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
     m = mn;
-    if (__any(smx >= sv_lim)) {  // a larger sigma than any before: the weights' scale moves
+    if (__any(smx >= sv_lim) || !__any(smx >= sv_low)) {
       smx = fmaxf(smx, __shfl_xor(smx, 16, kWave));
       smx = fmaxf(smx, __shfl_xor(smx, 32, kWave));
-      const int e = norm_exp(__float_as_uint(smx));
-      if (sv_lim > 0.0f) f *= ldexpf(1.0f, e - sv_exp);
-      sv_exp = e;
-      sv_lim = ldexpf(1.0f, 15 - e);
+      // (The same in all lanes: the scale stays in scalar registers.)
+      const uint32_t top = __builtin_amdgcn_readfirstlane(__float_as_uint(smx));
+      if (top != 0) {  // (a tile of zeros weighs nothing at any scale)
+        const int e = min(norm_exp(top), sv_top);
+        f *= ldexpf(1.0f, e - sv_exp);
+        sv_exp = e;
+        sv_top = min(sv_top, e + 64);
+        sv_lim = pow2(15 - e);
+        sv_low = pow2(15 - 8 - e);
+      }
     }
     l *= f;
 #pragma unroll

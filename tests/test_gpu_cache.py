@@ -440,6 +440,78 @@ def test_codebook_decode_tiles(T, D, G, N, bits_k, bits_v, m, mag):
                mean_abs=1e-5)
 
 
+def _codebook_decode(T, q, R, ck, cv, kc, ks, vc, vs, n):
+    """tqkv_decode_attend_codebook over whole buffers: (out bf16 [B, H, D],
+    the merged f32 rows [B, H, D] in the rotated basis, which the call leaves
+    at the workspace's start)."""
+    B, H, D = q.shape
+    Hkv, cap = kc.shape[1], kc.shape[2]
+    bits = [int(np.log2(len(c))) for c in (ck, cv)]
+    d = [T.DeviceArray.of(np.ascontiguousarray(x)) for x in (q, R, ck, cv, kc, ks, vc, vs)]
+    out = T.DeviceArray((B, H, D), np.uint16)
+    ws = T.DeviceArray((T.decode_codebook_workspace_size(B, H, D, n) // 4,), np.float32)
+    T.decode_attend_codebook(d[0].ptr, B, H, Hkv, D, D ** -0.5, d[1].ptr, d[2].ptr, bits[0],
+                             d[3].ptr, bits[1], d[4].ptr, d[5].ptr, d[6].ptr, d[7].ptr, cap, n,
+                             out.ptr, ws.ptr, ws.numpy().nbytes)
+    T.hip().sync()
+    return out.numpy(), ws.numpy()[:B * H * D].reshape(B, H, D).copy()
+
+
+def _codebook_want(q, R, ck, cv, kc, ks, vc, vs, n):
+    """The same in 64 bits: (out, the rows in the rotated basis)."""
+    B, H, D = q.shape
+    G = H // kc.shape[1]
+    q64, R64 = O.bf16_to_f32(q).astype(np.float64), R.astype(np.float64)
+    rot = np.empty((B, H, D))
+    for b in range(B):
+        for h in range(H):
+            i = (b, h // G, slice(0, n))
+            k = ck.astype(np.float64)[kc[i]] * ks[i][:, None].astype(np.float64)
+            s = (k @ (R64 @ q64[b, h])) * D ** -0.5
+            p = np.exp(s - s.max())
+            p = p / p.sum() * vs[i].astype(np.float64)
+            rot[b, h] = np.where(p > 0, p, 0.0) @ cv.astype(np.float64)[vc[i]]
+    return rot @ R64, rot
+
+
+@pytest.mark.parametrize("D,G,bits", [(64, 2, 4), (128, 16, 8), (256, 2, 3), (256, 16, 4),
+                                      (512, 16, 4), (512, 4, 6)])
+@pytest.mark.parametrize("sigmas", ["zeros, then 1e-6", "zeros, then 1e-9", "shrinking",
+                                    "zeros between"])
+def test_codebook_decode_follows_the_value_sigmas(T, D, G, bits, sigmas):
+    """Value sigmas that differ by more than a weight's two f16 parts hold
+    together: tiles of zeros before small ones, a tile of far larger ones whose
+    tokens weigh nothing, zeros between. The error is the f32 sums' own."""
+    print(f"[codebook-sigmas] D={D} G={G} bits={bits} {sigmas}", flush=True)
+    B, Hkv, N = 1, 2, 400
+    rng = np.random.default_rng(D + G)
+    q = O.bf16_from_f32(np.repeat(rng.standard_normal((B, Hkv, D)).astype(np.float32), G, axis=1))
+    R, cent = T.rotation_matrix(D, 42), T.lloyd_max(bits, 100)[1].astype(np.float32)
+    kc, vc = (rng.integers(0, 1 << bits, (B, Hkv, N, D), dtype=np.uint8) for _ in "kv")
+    ks, vs = (rng.uniform(0.5, 2, (B, Hkv, N)).astype(np.float32) for _ in "kv")
+    first = 128  # a whole tile at every D
+    if sigmas == "shrinking":
+        # The first tile's keys are against the query: weights below e^-25.
+        vs *= 1e-5
+        vs[..., :first] *= 1e10
+        rot = O.bf16_to_f32(q[:, ::G]).astype(np.float64) @ R.T.astype(np.float64)
+        kc[:, :, :first] = np.where(rot > 0, 0, (1 << bits) - 1)[:, :, None]
+        ks[..., :first] = 6.0 if D == 64 else 2.0
+    else:
+        vs *= 1e-9 if "1e-9" in sigmas else 1e-6
+        vs[..., :first] = 0
+        if sigmas == "zeros between":
+            vs[..., :first] = 3e-6
+            vs[..., first:2 * first] = 0
+    got, merged = _codebook_decode(T, q, R, cent, cent, kc, ks, vc, vs, N)
+    want, rot = _codebook_want(q, R, cent, cent, kc, ks, vc, vs, N)
+    # f32 sums of D products in the scores, of N in the values.
+    err = np.abs(merged - rot).max() / np.sqrt(np.mean(rot ** 2))
+    print(f"[codebook-sigmas] merged rows: max error {err:.2e} of their rms", flush=True)
+    assert err < 1e-4
+    check_bf16(got, want, "codebook-sigmas", scale=np.abs(want).max(), max_abs=1e-4, mean_abs=1e-5)
+
+
 def test_codebook_decode_rejects_unaligned_values(T):
     """A lane loads its value codes 4 bytes at a time at D = 256: a value
     code pointer off that alignment is refused before any launch."""
