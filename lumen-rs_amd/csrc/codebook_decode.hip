@@ -19,7 +19,11 @@
 // heads take three products. A code is looked up once for all heads (one
 // 4-byte LDS read: hi | lo << 16), where f32 multiply-adds a head repeated
 // the lookups for every two heads at D = 512 and cost a vector operation a
-// code and head. Outputs are as far from 64 bits as before (half a bf16 step).
+// code and head. Against 64 bits the merged rows (before the rotation back and
+// the bf16 rounding) are 0.36 to 0.77 times as far off as that kernel's over 27
+// shapes of every head dim, width and head count (D = 512, 16 heads: 2.8e-6 ->
+// 1.2e-6; D = 64: 1.2e-6 -> 1.0e-6): the f32 chain over D channels had lost
+// more than the operands' last bits.
 // Measured a call: Gemma 4's global layers (B = 1, 32 / 2 heads, D = 512,
 // 32,768 tokens, 4-bit) 227 -> 43 us; B = 32, 16 / 8 heads, D = 256, 32,768
 // tokens, 3-bit 850 -> 803 us (5.4 TB/s; vector issue 68% of its cycles, LDS
@@ -123,12 +127,22 @@ struct Args {
 };
 
 // The power of two that puts values of magnitude up to the one with bits
-// `mx` into [2^14, 2^15) (1 for zero, infinity and NaN), as its exponent (at
-// most 90, so that sums of scaled weights stay finite).
+// `mx` into [2^14, 2^15), as its exponent (at most 90, so that sums of scaled
+// weights stay finite; 0 for zero, infinity and NaN).
 __device__ __forceinline__ int norm_exp(uint32_t mx) {
   const int e = int(mx >> 23) - 127;
   if (mx == 0 || e == 128) return 0;
   return 14 - e < 90 ? 14 - e : 90;
+}
+// The same for a whole operand (a table, a head's query): kWide where its
+// largest is an infinity, NaN or outside [2^-64, 2^64), which hi + lo does not
+// hold as f32 does. The decode then marks the head's partials (a sum of
+// kWideSum, which no sum of weights is) and the merge attends in f32.
+constexpr int kWide = 1 << 10;
+constexpr float kWideSum = -1.0f;
+__device__ __forceinline__ int operand_exp(uint32_t mx) {
+  const int e = int(mx >> 23) - 127;
+  return mx != 0 && (e < -64 || e > 63) ? kWide : norm_exp(mx);
 }
 __device__ __forceinline__ float pow2(int e) { return __uint_as_float(uint32_t(127 + e) << 23); }
 __device__ __forceinline__ uint32_t mag(float x) { return __float_as_uint(x) & 0x7fffffffu; }
@@ -265,7 +279,7 @@ void cb_decode_kernel(const Args a) {
       c[k] = 4 * lane + k < n ? cent[4 * lane + k] : 0.0f;
       mx = max(mx, mag(c[k]));
     }
-    const int e = norm_exp(largest(mx, kWave));
+    const int e = operand_exp(largest(mx, kWave));
     u4_t t;
 #pragma unroll
     for (int k = 0; k < 4; ++k) t[k] = split_h16(c[k] * pow2(e));
@@ -300,7 +314,7 @@ void cb_decode_kernel(const Args a) {
       v[k] = src[k];
       mx = max(mx, mag(v[k]));
     }
-    const int e = norm_exp(largest(mx, kLph));
+    const int e = operand_exp(largest(mx, kLph));
     if (h < G) {
       put_q(h, 2 * (i / 8) + i % 2, i / 2 % 4, v, e);
       if (i == 0) s_e[h] = e;
@@ -311,7 +325,7 @@ void cb_decode_kernel(const Args a) {
       const float* src = a.pq + (qrow + h) * a.qm;
       uint32_t mx = 0;
       for (int i = lane; i < a.qm; i += kWave) mx = max(mx, mag(src[i]));
-      const int e = norm_exp(largest(mx, kWave));
+      const int e = operand_exp(largest(mx, kWave));
       for (int i = lane; i < 4 * mk; i += kWave) {
         float v[8];
 #pragma unroll
@@ -553,34 +567,85 @@ void cb_decode_kernel(const Args a) {
     *reinterpret_cast<f4_t*>(po + 4 * r) = f4_t{o[0][r], o[1][r], o[2][r], o[3][r]};
   if (wave == 0 && lg == 0) {
     a.part_m[row] = m;
-    a.part_l[row] = ldexpf(l, -sv_exp);
+    const bool wide = s_e[hd] == kWide || (QJL && s_e[16 + hd] == kWide) || s_e[32] == kWide ||
+                      s_e[33] == kWide;
+    a.part_l[row] = wide ? kWideSum : ldexpf(l, -sv_exp);
   }
+}
+
+// Channel d of one (batch row, head)'s attention over all tokens, in f32 on
+// the vector units: for operands marked kWide, which no cache's own are
+// (Lloyd-Max centroids of a unit normal, bf16 queries of common sizes). A
+// wavefront: a lane a token for the scores, then a channel.
+__device__ float attend_f32(const Args& a, int64_t bh, int D, int d) {
+  const int lane = threadIdx.x;
+  const int64_t slab = bh / a.H * a.H_kv * a.cap + bh % a.H / a.G * a.cap;
+  const float *q = a.qs + bh * D, *pq = a.pq + bh * a.qm;
+  float m = -INFINITY, l = 0.0f, o = 0.0f;
+  for (int64_t base = 0; base < a.n; base += kWave) {
+    const int cnt = a.n - base < kWave ? int(a.n - base) : kWave;
+    const int64_t row = slab + base + lane;
+    float x = -INFINITY;
+    if (lane < cnt) {
+      x = 0.0f;
+      for (int i = 0; i < D; ++i) {
+        const int c = a.kc[row * D + i];
+        x = fmaf(q[i], c < a.n_k ? a.cent_k[c] : 0.0f, x);
+      }
+      x *= a.ks[row];
+      if (a.ksg && a.krn[row] >= 1e-10f) {
+        float c = 0.0f;
+        for (int i = 0; i < a.qm; ++i)
+          c += (a.ksg[row * ((a.qm + 31) / 32) + i / 32] >> (i % 32)) & 1u ? pq[i] : -pq[i];
+        x = fmaf(c * (a.krn[row] * (1.2533141373155001f / sqrtf(float(a.qm)))), a.qscale, x);
+      }
+    }
+    float mx = x;
+    for (int off = 1; off < kWave; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+    const float mn = fmaxf(m, mx);
+    const float f = m == -INFINITY ? 0.0f : exp2f(m - mn);
+    m = mn;
+    const float p = lane < cnt ? exp2f(x - (mn == -INFINITY ? 0.0f : mn)) : 0.0f;
+    const float w = lane < cnt ? p * a.vs[row] : 0.0f;
+    float ps = p;
+    for (int off = 1; off < kWave; off <<= 1) ps += __shfl_xor(ps, off, kWave);
+    l = l * f + ps;
+    o *= f;
+    for (int t = 0; t < cnt; ++t) {
+      const int c = a.vc[(slab + base + t) * D + d];
+      o = fmaf(__shfl(w, t, kWave), c < a.n_v ? a.cent_v[c] : 0.0f, o);
+    }
+  }
+  return l > 0.0f ? o / l : 0.0f;
 }
 
 // The splits of one (batch row, head) merged in the rotated basis: a thread a
 // channel, every split's partial loaded with no test between (an empty
 // weight is 0), so the loads issue together.
-__global__ __launch_bounds__(64) void cb_merge_kernel(const float* __restrict__ part_o,
-                                                      const float* __restrict__ part_m,
-                                                      const float* __restrict__ part_l,
-                                                      int n_splits, int D, float* __restrict__ o) {
+__global__ __launch_bounds__(64) void cb_merge_kernel(const Args a, int D, float* __restrict__ o) {
   __shared__ float s_w[64];
   const int64_t bh = blockIdx.x;
+  const int n_splits = a.n_splits;
   const int lane = threadIdx.x;  // n_splits <= 64: a lane a split, then a channel
-  const float pm = lane < n_splits ? part_m[bh * n_splits + lane] : -INFINITY;
+  const int d = int(blockIdx.y) * kWave + lane;
+  const float pm = lane < n_splits ? a.part_m[bh * n_splits + lane] : -INFINITY;
+  const float pl = lane < n_splits ? a.part_l[bh * n_splits + lane] : 0.0f;
+  if (__any(pl == kWideSum)) {
+    o[bh * D + d] = attend_f32(a, bh, D, d);
+    return;
+  }
   float mx = pm;
 #pragma unroll
   for (int off = 1; off < kWave; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
   const float w = pm != -INFINITY ? exp2f(pm - mx) : 0.0f;
   s_w[lane] = w;
-  float ls = lane < n_splits ? part_l[bh * n_splits + lane] * w : 0.0f;
+  float ls = pl * w;
 #pragma unroll
   for (int off = 1; off < kWave; off <<= 1) ls += __shfl_xor(ls, off, kWave);
   __syncthreads();
-  const int d = int(blockIdx.y) * kWave + lane;
   float os = 0.0f;
 #pragma unroll 16
-  for (int s = 0; s < n_splits; ++s) os += part_o[(bh * n_splits + s) * D + d] * s_w[s];
+  for (int s = 0; s < n_splits; ++s) os += a.part_o[(bh * n_splits + s) * D + d] * s_w[s];
   o[bh * D + d] = ls > 0.0f ? os / ls : 0.0f;
 }
 
@@ -738,7 +803,7 @@ int32_t decode_codebook(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, i
   TQKV_LAUNCHED();
   // The merged rows take the rotated query's place (its last reader has run).
   hipLaunchKernelGGL(cb::cb_merge_kernel, dim3(unsigned(qrows), unsigned(D / 64)), dim3(64), 0, st,
-                     po, pm, pl, n_splits, D, qr);
+                     a, D, qr);
   TQKV_LAUNCHED();
   cb::launch_matmul<false>(static_cast<const float*>(qr), rotation, D, D, qrows, 1.0f, nullptr,
                            nullptr, out, st);

@@ -379,6 +379,7 @@ def test_codebook_decode_direct(T, B, Hkv, G, D, N, bits):
     (128, 2, 65, 2, 2, 33, 0), (128, 4, 129, 3, 4, 0, 8), (128, 1, 700, 8, 8, 0, 0),
     (256, 2, 64, 3, 3, 64, 0), (256, 16, 513, 4, 4, 96, 8), (256, 8, 300, 6, 4, 0, 0),
     (512, 16, 127, 4, 4, 0, 8), (512, 4, 128, 4, 4, 1024, 0), (512, 16, 641, 7, 7, 40, 0),
+    (512, 16, 300, 4, 4, 1024, 0), (256, 16, 200, 8, 8, 1024, 0),  # the most LDS
     (512, 1, 130, 1, 1, 0, 0)])
 def test_codebook_decode_tiles(T, D, G, N, bits_k, bits_v, m, mag):
     """The decode's tile edges (64 tokens, 128 at D = 512), splits, head groups
@@ -510,6 +511,122 @@ def test_codebook_decode_follows_the_value_sigmas(T, D, G, bits, sigmas):
     print(f"[codebook-sigmas] merged rows: max error {err:.2e} of their rms", flush=True)
     assert err < 1e-4
     check_bf16(got, want, "codebook-sigmas", scale=np.abs(want).max(), max_abs=1e-4, mean_abs=1e-5)
+
+
+@pytest.mark.parametrize("D,G,bits,m", [(64, 8, 4, 0), (128, 2, 8, 40), (256, 16, 3, 0),
+                                        (512, 1, 4, 33), (512, 16, 6, 0)])
+@pytest.mark.parametrize("what", ["key centroids", "value centroids", "small tables", "query"])
+def test_codebook_decode_operands_beyond_two_f16_parts(T, D, G, bits, m, what):
+    """Infinite centroids, and tables and queries so large or small that their
+    f16 parts cannot be brought to one scale: the results of f32 arithmetic.
+    Key centroids: -infinity makes a token weigh nothing. Value centroids:
+    +infinity makes every output infinite, of the rotation's sign."""
+    print(f"[codebook-wide] D={D} G={G} bits={bits} m={m} {what}", flush=True)
+    B, Hkv, N = 2, 2, 300
+    rng = np.random.default_rng(D + G + bits)
+    q = O.bf16_from_f32(np.repeat(rng.standard_normal((B, Hkv, D)).astype(np.float32), G, axis=1))
+    R, cent = T.rotation_matrix(D, 42), T.lloyd_max(bits, 100)[1].astype(np.float32)
+    ck, cv, top = cent.copy(), cent.copy(), (1 << bits) - 1
+    kc, vc = (rng.integers(0, top, (B, Hkv, N, D), dtype=np.uint8) for _ in "kv")  # no `top` yet
+    ks, vs = (rng.uniform(0.5, 2, (B, Hkv, N)).astype(np.float32) for _ in "kv")
+    rot = O.bf16_to_f32(q[:, ::G]).astype(np.float64) @ R.T.astype(np.float64)
+    mask = np.zeros((B, Hkv, N), bool)
+    d = np.argmax(np.abs(rot), axis=-1)
+    if what == "key centroids":
+        ck[top] = -np.inf
+        for b in range(B):
+            for h in range(Hkv):
+                d[b, h] = np.argmax(rot[b, h])  # there the query is positive
+                kc[b, h, 5::7, d[b, h]] = top
+                mask[b, h, 5::7] = True
+    elif what == "value centroids":
+        cv[top] = np.inf
+        for b in range(B):
+            for h in range(Hkv):
+                vc[b, h, 200, d[b, h]] = top
+    elif what == "small tables":
+        ck, cv = ck * np.float32(2.0 ** -100), cv * np.float32(2.0 ** 90)
+        ks, vs = ks * np.float32(2.0 ** 100), vs * np.float32(2.0 ** -90)
+    else:
+        q = O.bf16_from_f32(O.bf16_to_f32(q) * np.float32(2.0 ** 70))
+        ks = ks * np.float32(2.0 ** -70)
+    signs = rng.integers(0, 1 << 32, (B, Hkv, N, (m + 31) // 32), dtype=np.uint32)
+    rn = rng.uniform(0.1, 1, (B, Hkv, N)).astype(np.float32)
+    if what == "query":  # (norms below 1e-10 take no correction)
+        rn = rn * np.float32(2.0 ** -70)
+    phi = (rng.standard_normal((max(m, 1), D)) / np.sqrt(max(m, 1))).astype(np.float32)
+    H = G * Hkv
+    x = [T.DeviceArray.of(np.ascontiguousarray(a)) for a in
+         (q, R, ck, cv, kc, ks, vc, vs, signs if m else rn, rn, phi)]
+    out = T.DeviceArray((B, H, D), np.uint16)
+    head = (x[0].ptr, B, H, Hkv, D, D ** -0.5, x[1].ptr, x[2].ptr, bits, x[3].ptr, bits)
+    tail = (x[6].ptr, x[7].ptr, N, N, out.ptr, None, 0, None)
+    if m:
+        T.check(T.lib().tqkv_decode_attend_codebook_qjl(*head, x[4].ptr, x[5].ptr, x[8].ptr,
+                                                        x[9].ptr, x[10].ptr, m, *tail))
+    else:
+        T.decode_attend_codebook(*head, x[4].ptr, x[5].ptr, *tail)
+    T.hip().sync()
+    got = O.bf16_to_f32(out.numpy())
+    if what == "value centroids":
+        sign = np.sign(R[d.reshape(-1)]).reshape(B, Hkv, D)
+        assert np.array_equal(got, np.repeat(np.where(sign > 0, np.inf, -np.inf), G, axis=1))
+        return
+    q64, R64 = O.bf16_to_f32(q).astype(np.float64), R.astype(np.float64)
+    want = np.empty((B, H, D))
+    for b in range(B):
+        for h in range(H):
+            i = (b, h // G)
+            k = np.where(mask[i][:, None], 0.0, np.where(np.isfinite(ck), ck, 0).astype(np.float64)[kc[i]])
+            s = k * ks[i][:, None].astype(np.float64) @ (R64 @ q64[b, h])
+            if m:
+                bit = (signs[i][:, np.arange(m) // 32] >> (np.arange(m) % 32).astype(np.uint32)) & 1
+                s = s + np.where(rn[i] >= 1e-10, rn[i], 0) * np.sqrt(np.pi / 2) / np.sqrt(m) * (
+                    (2.0 * bit - 1) @ (phi.astype(np.float64) @ q64[b, h]))
+            s = np.where(mask[i], -np.inf, s * D ** -0.5)
+            p = np.exp(s - s.max())
+            want[b, h] = (p / p.sum() * vs[i]) @ cv.astype(np.float64)[vc[i]] @ R64
+    check_bf16(out.numpy(), want, "codebook-wide", scale=np.abs(want).max(), max_abs=1e-4,
+               mean_abs=1e-5)
+
+
+def test_codebook_decode_infinite_value_sigma(T):
+    """A token of infinite value sigma: the rotation back adds infinities of
+    both signs, NaN, in its heads alone."""
+    B, Hkv, G, D, N, bits = 1, 2, 4, 128, 200, 4
+    rng = np.random.default_rng(8)
+    q = O.bf16_from_f32(rng.standard_normal((B, Hkv * G, D)).astype(np.float32))
+    R, cent = T.rotation_matrix(D, 42), T.lloyd_max(bits, 100)[1].astype(np.float32)
+    kc, vc = (rng.integers(0, 1 << bits, (B, Hkv, N, D), dtype=np.uint8) for _ in "kv")
+    ks, vs = (rng.uniform(0.5, 2, (B, Hkv, N)).astype(np.float32) for _ in "kv")
+    vs[0, 1, 77] = np.inf
+    got = O.bf16_to_f32(_codebook_decode(T, q, R, cent, cent, kc, ks, vc, vs, N)[0])
+    want = _codebook_want(q, R, cent, cent, kc, ks, vc, np.where(np.isinf(vs), 0, vs), N)[0]
+    assert np.isnan(got[:, G:]).all()
+    check_bf16(O.bf16_from_f32(got[:, :G]), want[:, :G], "codebook-inf")
+
+
+@pytest.mark.parametrize("D,G,bits,N", [(64, 4, 4, 3000), (128, 1, 2, 2000), (128, 4, 8, 1500),
+                                        (256, 2, 3, 4000), (256, 16, 3, 1000), (512, 16, 4, 2000),
+                                        (512, 8, 6, 700)])
+def test_codebook_decode_holds_f32_precision(T, D, G, bits, N):
+    """The merged rows before the rotation back and the bf16 rounding, against
+    64 bits: the kernel's operands are two f16 parts each, and its error must
+    be that of f32 sums. An f32 multiply-add chain over the D channels of a
+    score (unit roundoff 2^-24) put the rows 0.5e-6 (D = 64) to 2.8e-6 (D =
+    512) off at such shapes; the bar is 2^-23 sqrt(D), 0.95e-6 to 2.7e-6."""
+    B, Hkv = 2, 2
+    rng = np.random.default_rng(D + bits)
+    q = O.bf16_from_f32(2 * rng.standard_normal((B, Hkv * G, D)).astype(np.float32))
+    R, cent = T.rotation_matrix(D, 42), T.lloyd_max(bits, 100)[1].astype(np.float32)
+    kc, vc = (np.searchsorted((cent[1:] + cent[:-1]) / 2, rng.standard_normal((B, Hkv, N, D)))
+              .astype(np.uint8) for _ in "kv")
+    ks, vs = (rng.uniform(0.5, 2, (B, Hkv, N)).astype(np.float32) for _ in "kv")
+    _, merged = _codebook_decode(T, q, R, cent, cent, kc, ks, vc, vs, N)
+    _, rot = _codebook_want(q, R, cent, cent, kc, ks, vc, vs, N)
+    rel = np.linalg.norm(merged - rot) / np.linalg.norm(rot)
+    print(f"[codebook-f32] D={D} G={G} bits={bits} N={N}: {rel:.2e}", flush=True)
+    assert rel <= 2.0 ** -23 * np.sqrt(D)
 
 
 def test_codebook_decode_rejects_unaligned_values(T):
