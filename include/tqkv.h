@@ -372,9 +372,9 @@ int32_t tqkv_decode_attend_codebook_qjl(const uint16_t* q, int32_t B, int32_t H,
  * dequantize as mlx::dequantize does for bf16 (bf16(fma(scale, code,
  * bias)), one rounding), then attention runs with bf16 operands and f32 accumulation. When
  * 8 or more row blocks share a KV head (fewer at D = 256 and 512), the
- * keys are dequantized once into the library's per-device scratch (2 * B *
- * H_kv * keys * D * 2 bytes, at most 4 GiB; larger contexts dequantize in
- * every block instead, in LDS) and read from there; the two ways give the
+ * keys that the chunk sees are dequantized once into the library's per-device
+ * scratch (2 * B * H_kv * keys * D * 2 bytes, at most 4 GiB; more keys are
+ * dequantized in every block instead, in LDS) and read from there; the two ways give the
  * same bits. A chunk with too few row blocks to fill the GPU over more than
  * 1,024 keys that it can see splits the keys over workgroups, their partials
  * in the same scratch, and merges them (f32, so apart from the unsplit sums

@@ -28,7 +28,8 @@ KernelFn pick(int D, int bk, int bv, bool h16 = false) {
   return nullptr;
 }
 
-// Dequantize-once: keys [0, total) of every (batch row, KV head), K into kd
+// Dequantize-once: keys [0, total) of every (batch row, KV head) (of segments
+// that start at the first visible tile, see keys_from), K into kd
 // as bf16 rows [B * H_kv, slab_rows, D] with mlx::dequantize's arithmetic
 // (bf16(fma(scale, code, bias)), one rounding), V into vd as the prefill
 // kernel's V operands (those bf16 values times 2^-kVShift, in f16; see
@@ -156,13 +157,21 @@ void launch_dequantize_rows(const Args& a, int bits, int kinds, int64_t slab_row
 #undef TQKV_DQ
 }
 
-// Rows a slab of the dequantize-once scratch holds: total, padded to whole
-// 64-key tiles where V is tiled (width kPreF16T; K shares the stride).
-int64_t once_slab_rows(bool tiled, int64_t total) {
-  return tiled ? (total + kTile - 1) / kTile * kTile : total;
-}
-size_t once_bytes(int64_t slabs, int64_t slab_rows, int D) {
-  return 2 * size_t(slabs) * size_t(slab_rows) * size_t(D) * 2;
+// a's keys [lo, lo + keys) alone: its segments start at key lo.
+Args keys_from(const Args& a, int D, int bk, int bv, int64_t lo, int64_t keys) {
+  Args k = a;
+  const int i = lo < a.n0 ? 0 : 1;
+  const int64_t skip = i ? lo - a.n0 : lo;
+  Seg& s = k.seg[i];
+  s.kw += skip * (int64_t(D) * bk / 32);
+  s.vw += skip * (int64_t(D) * bv / 32);
+  s.ks += skip * (D / a.gs);
+  s.kb += skip * (D / a.gs);
+  s.vs += skip * (D / a.gs);
+  s.vb += skip * (D / a.gs);
+  k.n0 = i ? 0 : a.n0 - lo;
+  k.total = keys;
+  return k;
 }
 
 // Both halves of the dequantize-once pass: one launch when K and V share a
@@ -170,7 +179,7 @@ size_t once_bytes(int64_t slabs, int64_t slab_rows, int D) {
 template <int D>
 void dequantize_rows(const Args& a, int bk, int bv, int64_t slabs, bool tiled, hipStream_t st,
                      uint16_t* kd, uint16_t* vd) {
-  const int64_t sr = once_slab_rows(tiled, a.total);
+  const int64_t sr = prefillplan::once_slab_rows(tiled, a.total);
   // (Tiled V: whole 64-key blocks, so that every tile is written.)
   const unsigned chunks = unsigned((sr * (D / 32) + 255) / 256);
   const int vt = tiled ? 1 : 0;
@@ -181,21 +190,6 @@ void dequantize_rows(const Args& a, int bk, int bv, int64_t slabs, bool tiled, h
     launch_dequantize_rows<D>(a, bv, 2, sr, vt, dim3(chunks, unsigned(slabs), 1), st, kd, vd);
   }
 }
-
-// Row blocks sharing one (batch row, KV head) from which the keys are
-// dequantized once into scratch instead of in every block: the blocks would
-// otherwise repeat the same dequantization, the kernel's VALU-bound part.
-// The wide kernel takes fewer: at D = 512 any (the in-block kernel spills;
-// 16 / 4 heads, 94 rows over 1,117 keys: 131 us in block, 44 once), at D = 256
-// half as many over 2,048 keys or more (B = 4, 16 / 8 heads, 300 rows over
-// 3,000 keys: 132 us in block, 107 once; 298 rows over 809: 35 and 42).
-constexpr int64_t kOnceBlocks = 8;
-int64_t once_blocks(int D, int64_t total) {
-  return D == 512 ? 1 : D == 256 && total >= 2048 ? 4 : kOnceBlocks;
-}
-// The scratch that path may take (bf16 K and V of every visible key); larger
-// contexts dequantize in every block instead.
-constexpr size_t kOnceMaxBytes = size_t(4) << 30;
 
 // The splits' partials of each row (slots (row, split), row = (b L + l) H +
 // h) combined and written as bf16: four channels a thread.
@@ -442,8 +436,9 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   const int64_t blocks = (int64_t(L) * a.G + rows_per_block - 1) / rows_per_block;
   if (blocks * H_kv * B > 0x7fffffff) return fail(TQKV_EINVAL_SHAPE, "grid too large");
   const int64_t units = blocks * H_kv * B, q_rows = int64_t(B) * H * L;
+  const size_t ws_bytes = workspace ? workspace_bytes : 0;
   const prefillplan::Chunk chunk{B, H, H_kv, L, D, a.total, q_start, k_start, a.causal != 0,
-                                 a.window, blocks, bf16_rows, library_scratch};
+                                 a.window, blocks, bf16_rows, library_scratch, ws_bytes};
   size_t part_bytes = 0;
   const auto use_splits = [&](const prefillplan::Splits& sp) {
     a.n_splits = a.n_part = int(sp.n);
@@ -468,57 +463,48 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   // TQKV_PREFILL_DEQUANT_ONCE=0 / 1 forces the choice (tests compare them).
   const char* once_env = getenv("TQKV_PREFILL_DEQUANT_ONCE");
   const int64_t slabs = int64_t(B) * H_kv;
-  // V as transposed tiles: always at D = 128; at D = 256 and 512 (the wide
-  // kernel) wherever the scratch has room for whole tiles, which the
-  // library's own has and a caller's workspace of
-  // tqkv_prefill_workspace_size bytes has for whole numbers of 64 keys.
-  const size_t tiled_bytes = once_bytes(slabs, once_slab_rows(true, a.total), D);
-  const bool tiled = D == 128 || (D > 128 && (library_scratch || workspace_bytes >= tiled_bytes));
-  const int64_t slab_rows = once_slab_rows(tiled, a.total);
-  const size_t need = once_bytes(slabs, slab_rows, D);
-  // With a caller workspace (the _ws entry) the dequantized rows go there
-  // when it holds them, else every block dequantizes for itself.
-  const bool fits = library_scratch || (workspace && workspace_bytes >= need);
-  bool once = !bf16_rows && fits &&
-              (once_env ? strcmp(once_env, "0") != 0
-                        : blocks >= once_blocks(D, a.total) &&
-                              once_bytes(slabs, a.total, D) <= kOnceMaxBytes);
+  const prefillplan::Once rows =
+      prefillplan::dequantize_once(chunk, once_env ? strcmp(once_env, "0") != 0 : -1);
+  bool once = rows.on;
   // Scratch that the call could do without (the partials; the rows of few
   // blocks) is left out where the library's cannot grow.
   void* ws = workspace;
   if (library_scratch && (once || part_bytes)) {
-    const size_t rows_bytes = once ? need : 0;
-    bool held = part_bytes && scratch_optional(rows_bytes + part_bytes, st, &ws);
+    bool held = part_bytes && scratch_optional((once ? rows.bytes : 0) + part_bytes, st, &ws);
     if (!held) use_splits(prefillplan::no_splits(chunk));
     if (once && !held) {
-      if (blocks >= kOnceBlocks || once_env) {
-        if (int32_t rc = scratch_for_current_device(need, &ws)) return rc;
+      if (blocks >= prefillplan::kOnceBlocks || once_env) {
+        if (int32_t rc = scratch_for_current_device(rows.bytes, &ws)) return rc;
       } else {
-        once = scratch_optional(need, st, &ws);
+        once = scratch_optional(rows.bytes, st, &ws);
       }
     }
   }
   const int64_t grid = units * a.n_splits;
   if (once) {
     uint16_t* kd = static_cast<uint16_t*>(ws);
-    uint16_t* vd = kd + size_t(slabs) * size_t(slab_rows) * size_t(D);
+    uint16_t* vd = kd + size_t(slabs) * size_t(rows.slab_rows) * size_t(D);
     if (slabs > 65535) return fail(TQKV_EINVAL_SHAPE, "B * H_kv = %lld slabs", (long long)slabs);
+    const Args d = keys_from(a, D, bits_k, bits_v, rows.lo, rows.keys);
     switch (D) {
-      case 64: dequantize_rows<64>(a, bits_k, bits_v, slabs, tiled, st, kd, vd); break;
-      case 128: dequantize_rows<128>(a, bits_k, bits_v, slabs, tiled, st, kd, vd); break;
-      case 256: dequantize_rows<256>(a, bits_k, bits_v, slabs, tiled, st, kd, vd); break;
-      default: dequantize_rows<512>(a, bits_k, bits_v, slabs, tiled, st, kd, vd); break;
+      case 64: dequantize_rows<64>(d, bits_k, bits_v, slabs, rows.tiled, st, kd, vd); break;
+      case 128: dequantize_rows<128>(d, bits_k, bits_v, slabs, rows.tiled, st, kd, vd); break;
+      case 256: dequantize_rows<256>(d, bits_k, bits_v, slabs, rows.tiled, st, kd, vd); break;
+      default: dequantize_rows<512>(d, bits_k, bits_v, slabs, rows.tiled, st, kd, vd); break;
     }
     TQKV_LAUNCHED();
     Args p = a;
     const uint16_t* none = kd;  // scales and biases: never read at this width
     p.seg[0] = Seg{reinterpret_cast<const uint32_t*>(kd), none, none,
-                   reinterpret_cast<const uint32_t*>(vd), none, none, slab_rows,
-                   int64_t(H_kv) * slab_rows};
+                   reinterpret_cast<const uint32_t*>(vd), none, none, rows.slab_rows,
+                   int64_t(H_kv) * rows.slab_rows};
     p.seg[1] = p.seg[0];
-    p.n0 = a.total;
-    if (part_bytes) use_parts(p, static_cast<char*>(ws) + need);
-    if (D >= 256 && tiled) {
+    // (The splits start at the first visible tile too.)
+    p.n0 = p.total = rows.keys;
+    p.k_start = a.k_start + rows.lo;
+    p.split_lo = 0;
+    if (part_bytes) use_parts(p, static_cast<char*>(ws) + rows.bytes);
+    if (D >= 256 && rows.tiled) {
       // Rows a block by rounds of workgroups over the CUs (one a CU), a 64-row
       // block's taking 0.87 of a 128-row one's time (32 / 2 heads, D = 512,
       // 512 rows over 8,192 keys, one round each: 331 and 380 us).
@@ -531,7 +517,7 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
       hipLaunchKernelGGL(pick_wide(D, wide_rows), dim3(unsigned(p.n_blocks * per_block)),
                          dim3(4 * wide_rows), 0, st, p);
     } else {
-      hipLaunchKernelGGL(pick(D, kPreBits, tiled ? kPreF16T : kPreF16), dim3(unsigned(grid)),
+      hipLaunchKernelGGL(pick(D, kPreBits, rows.tiled ? kPreF16T : kPreF16), dim3(unsigned(grid)),
                          dim3(threads), 0, st, p);
     }
     TQKV_LAUNCHED();
@@ -567,7 +553,8 @@ extern "C" int32_t tqkv_prefill_attend_affine(const uint16_t* q, int32_t B, int3
 extern "C" size_t tqkv_prefill_workspace_size(int32_t B, int32_t H_kv, int32_t D,
                                               int64_t total_keys) {
   if (B <= 0 || H_kv <= 0 || D <= 0 || total_keys <= 0) return 0;
-  return once_bytes(int64_t(B) * H_kv, once_slab_rows(D == 128, total_keys), D);
+  return prefillplan::once_bytes(int64_t(B) * H_kv,
+                                 prefillplan::once_slab_rows(D == 128, total_keys), D);
 }
 
 extern "C" int32_t tqkv_prefill_attend_affine_ws(

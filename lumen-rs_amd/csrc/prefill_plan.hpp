@@ -20,6 +20,7 @@ struct Chunk {
   int64_t blocks;        // row blocks a KV head in the in-block kernel
   bool bf16_rows;        // K and V are bf16 rows, not packed codes
   bool library_scratch;  // else a caller's workspace, which holds rows only
+  size_t ws_bytes;       // of that workspace
 };
 
 // The keys [lo, hi] that some row of the chunk sees, lo down to a whole tile;
@@ -35,6 +36,64 @@ inline Visible visible_keys(const Chunk& c) {
       lo = c.q_start - c.window + 1 - c.k_start;
   }
   return Visible{lo / kTileKeys * kTileKeys, hi};
+}
+
+// Bytes of the dequantized K and V rows of every (batch row, KV head).
+inline size_t once_bytes(int64_t slabs, int64_t slab_rows, int64_t D) {
+  return 2 * size_t(slabs) * size_t(slab_rows) * size_t(D) * 2;
+}
+// Rows a slab of them holds: the keys, up to whole tiles where V is tiled (K
+// shares the stride).
+inline int64_t once_slab_rows(bool tiled, int64_t keys) {
+  return tiled ? (keys + kTileKeys - 1) / kTileKeys * kTileKeys : keys;
+}
+
+// Row blocks sharing one (batch row, KV head) from which its visible keys are
+// dequantized once into scratch instead of in every block: the blocks would
+// otherwise repeat the same dequantization, the kernel's VALU-bound part.
+// The wide kernel takes fewer: at D = 512 any (the in-block kernel spills;
+// 16 / 4 heads, 94 rows over 1,117 keys: 131 us in block, 44 once; 32 / 2
+// heads, 4 rows over 64 keys: 21.1 and 16.5), at D = 256
+// half as many over 2,048 keys or more (B = 4, 16 / 8 heads, 300 rows over
+// 3,000 keys: 132 us in block, 107 once; 298 rows over 809: 35 and 42).
+// Only the keys that the chunk sees are dequantized and counted: of 65,536
+// keys under a window of 1,024, 300 rows take 47 us at D = 256 (16 / 8 heads)
+// and 67 at D = 512 (32 / 2); with all keys 154 and 121.
+constexpr int64_t kOnceBlocks = 8;
+inline int64_t once_blocks(int64_t D, int64_t keys) {
+  return D == 512 ? 1 : D == 256 && keys >= 2048 ? 4 : kOnceBlocks;
+}
+// The scratch that path may take; more keys dequantize in every block instead.
+constexpr size_t kOnceMaxBytes = size_t(4) << 30;
+
+// Dequantize once: keys [lo, lo + keys) as slabs of slab_rows rows, V as
+// transposed tiles where `tiled`.
+struct Once {
+  bool on = false;
+  int64_t lo = 0, keys = 0, slab_rows = 0;
+  bool tiled = false;
+  size_t bytes = 0;
+};
+// force: 0 or 1 (tests compare the two ways), -1 for the rule.
+inline Once dequantize_once(const Chunk& c, int force) {
+  Once o;
+  const Visible v = visible_keys(c);
+  o.lo = v.lo;
+  o.keys = v.hi - v.lo + 1;
+  if (c.bf16_rows || force == 0 || o.keys <= 0) return o;
+  // V as transposed tiles: always at D = 128; at D = 256 and 512 (the wide
+  // kernel) wherever there is room for whole tiles, which a caller's workspace
+  // sized for rows alone may not have.
+  const int64_t slabs = c.B * c.H_kv;
+  o.tiled = c.D == 128 ||
+            (c.D > 128 && (c.library_scratch ||
+                           c.ws_bytes >= once_bytes(slabs, once_slab_rows(true, o.keys), c.D)));
+  o.slab_rows = once_slab_rows(o.tiled, o.keys);
+  o.bytes = once_bytes(slabs, o.slab_rows, c.D);
+  if (!c.library_scratch && c.ws_bytes < o.bytes) return o;
+  o.on = force == 1 || (c.blocks >= once_blocks(c.D, o.keys) &&
+                        once_bytes(slabs, o.keys, c.D) <= kOnceMaxBytes);
+  return o;
 }
 
 // Key splits of a chunk whose row blocks would leave CUs idle (a short chunk

@@ -5,10 +5,10 @@
 using namespace tqkv::prefillplan;
 
 // c: B, H, H_kv, L, D, total, q_start, k_start, causal, window, blocks,
-// bf16_rows, library_scratch.
+// bf16_rows, library_scratch, ws_bytes.
 static Chunk chunk(const int64_t* c) {
   return Chunk{c[0], c[1], c[2], c[3], c[4],  c[5],       c[6],
-               c[7], c[8] != 0, c[9], c[10], c[11] != 0, c[12] != 0};
+               c[7], c[8] != 0, c[9], c[10], c[11] != 0, c[12] != 0, size_t(c[13])};
 }
 
 extern "C" {
@@ -25,5 +25,15 @@ void planhost_splits(const int64_t* c, int64_t* out) {
   out[1] = s.len;
   out[2] = s.lo;
   out[3] = int64_t(s.bytes);
+}
+// out: on, lo, keys, slab_rows, tiled, bytes.
+void planhost_once(const int64_t* c, int64_t force, int64_t* out) {
+  const Once o = dequantize_once(chunk(c), int(force));
+  out[0] = o.on;
+  out[1] = o.lo;
+  out[2] = o.keys;
+  out[3] = o.slab_rows;
+  out[4] = o.tiled;
+  out[5] = int64_t(o.bytes);
 }
 }

@@ -360,3 +360,68 @@ def test_prefill_with_caller_workspace(T, monkeypatch, N):
                                    None if ws is None else ws.ptr, ws_bytes, N - L, 0, True, -1)
         T.hip().sync()
         assert np.array_equal(out.numpy(), want), f"workspace of {ws_bytes} bytes"
+
+
+@pytest.mark.parametrize("P,S,L,window,D,H,Hkv,bk,bv,gs", [
+    (300, 1200, 512, 100, 128, 16, 4, 8, 4, 64),   # the first visible key in the suffix
+    (1000, 333, 200, 500, 128, 8, 2, 3, 6, 32),    # in the prefix
+    (1000, 333, 200, 500, 64, 8, 2, 4, 8, 64),
+    (640, 500, 130, 150, 256, 8, 4, 5, 4, 128),    # a tile past the seam
+    (900, 400, 90, 220, 512, 8, 1, 4, 4, 64),
+    (64, 900, 300, 64, 512, 8, 4, 6, 3, 64)])
+def test_prefill_dequantizes_the_visible_keys_of_both_segments(T, monkeypatch, P, S, L, window, D,
+                                                               H, Hkv, bk, bv, gs):
+    # A window over a shared prefix and suffixes: the dequantize-once pass
+    # starts at the first visible tile, in either segment. The same bits as in
+    # every block, with the library's scratch and a workspace, and the oracle's.
+    print(f"[prefill-visible] P={P} S={S} L={L} window={window} D={D}", flush=True)
+    B = 2
+    q = kv_bf16((B, H, L, D), P)
+    kp, vp = (kv_bf16((1, Hkv, P, D), P + i, frac=0.01, mult=10.0) for i in (1, 2))
+    ks, vs = (kv_bf16((B, Hkv, S, D), P + i, frac=0.01, mult=10.0) for i in (3, 4))
+    (kph, kpd), (vph, vpd) = _cache(kp, gs, bk, P + 7), _cache(vp, gs, bv, P + 7)
+    (ksh, ksd), (vsh, vsd) = _cache(ks, gs, bk, S + 3), _cache(vs, gs, bv, S + 3)
+    segs_host = [(kpd, vpd, P + 7, P, True), (ksd, vsd, S + 3, S, False)]
+    args = (B, H, Hkv, L, D, gs, bk, bv, D ** -0.5)
+    got = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("TQKV_PREFILL_DEQUANT_ONCE", mode)
+        got[mode] = run(T, q, segs_host, *args, P + S - L, 0, True, window)
+    assert np.array_equal(got["0"], got["1"])
+    seen = min(P + S, L + window)
+    dq = T.DeviceArray.of(q)
+    segs = [T.affine_seg(tuple(a.ptr for a in k), tuple(a.ptr for a in v), c, n, sh)
+            for (k, v, c, n, sh) in segs_host]
+    for rows in (seen + 63, (seen + 126) // 64 * 64):
+        wsb = 4 * B * Hkv * rows * D
+        ws = T.DeviceArray((wsb,), np.uint8, np.full((wsb,), 0xFF, np.uint8))
+        out = T.DeviceArray((B, H, L, D), np.uint16)
+        T.prefill_attend_affine_ws(dq.ptr, *args, segs, out.ptr, ws.ptr, wsb, P + S - L, 0, True,
+                                   window)
+        T.hip().sync()
+        assert np.array_equal(out.numpy(), got["0"]), f"workspace of {rows} rows a slab"
+    cat = lambda a, b: np.concatenate([np.broadcast_to(a, (B,) + a.shape[1:]), b], axis=2)
+    want = want_mlx(q, tuple(cat(a, b) for a, b in zip(kph, ksh)),
+                    tuple(cat(a, b) for a, b in zip(vph, vsh)), gs, bk, bv, D ** -0.5, causal=True,
+                    q_start=P + S - L, first_held=0, window=window)
+    check(got["1"], want, "visible keys")
+
+
+@pytest.mark.parametrize("D", [256, 512])
+def test_prefill_window_over_a_long_cache_holds_little_scratch(T, monkeypatch, D):
+    # 300 rows that see 1,000 of 20,000 keys: the visible keys' rows and the
+    # partials of two splits, not the whole cache's rows.
+    monkeypatch.delenv("TQKV_PREFILL_DEQUANT_ONCE", raising=False)
+    B, H, Hkv, L, N, window = 1, 8, 4, 300, 20000, 700
+    q = kv_bf16((B, H, L, D), 1)
+    k, v = (kv_bf16((B, Hkv, N, D), i) for i in (2, 3))
+    (kh, kd), (vh, vd) = _cache(k, 64, 4, N), _cache(v, 64, 4, N)
+    T.scratch_release()
+    got = run(T, q, [(kd, vd, N, N, False)], B, H, Hkv, L, D, 64, 4, 4, D ** -0.5, N - L, 0, True,
+              window)
+    assert T.scratch_bytes() <= 4 * B * Hkv * N * D / 4
+    keep = slice(N - 1088, N)
+    cut = lambda t: tuple(np.ascontiguousarray(a[:, :, keep]) for a in t)
+    want = want_mlx(q, cut(kh), cut(vh), 64, 4, 4, D ** -0.5, causal=True, q_start=1088 - L,
+                    first_held=0, window=window)
+    check(got, want, "window")

@@ -11,7 +11,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BUILD = os.path.join(ROOT, "tests", "_build")
 LIB = os.path.join(BUILD, "libprefillplanhost.so")
 FIELDS = ("B", "H", "Hkv", "L", "D", "total", "q_start", "k_start", "causal", "window", "blocks",
-          "bf16_rows", "library_scratch")
+          "bf16_rows", "library_scratch", "ws_bytes")
 ROWS = {64: 128, 128: 256, 256: 128, 512: 64}  # rows a block of the in-block kernel
 
 
@@ -24,10 +24,15 @@ def host():
     return ctypes.CDLL(LIB)
 
 
-def ask(fn, c, n):
+def ask(fn, c, n, *more):
     out = (ctypes.c_int64 * n)()
-    fn((ctypes.c_int64 * len(FIELDS))(*(int(c[f]) for f in FIELDS)), out)
+    fn((ctypes.c_int64 * len(FIELDS))(*(int(c[f]) for f in FIELDS)), *map(ctypes.c_int64, more), out)
     return list(out)
+
+
+def once(host, c, force=-1):
+    return dict(zip(("on", "lo", "keys", "slab_rows", "tiled", "bytes"),
+                    ask(host.planhost_once, c, 6, force)))
 
 
 def chunk(rng, **fixed):
@@ -39,7 +44,7 @@ def chunk(rng, **fixed):
     c = dict(B=rng.choice((1, 1, 2, 5)), H=Hkv * G, Hkv=Hkv, L=L, D=D, total=total,
              k_start=rng.choice((0, 0, 40, 100000)), causal=rng.random() < 0.8,
              window=rng.choice((-1, -1, 1, 100, 1500, 1 << 40)), bf16_rows=False,
-             library_scratch=rng.random() < 0.8)
+             library_scratch=rng.random() < 0.8, ws_bytes=0)
     c["q_start"] = rng.choice((c["k_start"] + total - L, 0, c["k_start"] + total // 2))
     c.update(fixed)
     c["blocks"] = -(-c["L"] * (c["H"] // c["Hkv"]) // ROWS[c["D"]])
@@ -101,3 +106,46 @@ def test_bf16_rows_are_never_split(host):
         for _ in range(500):
             n, _, lo, size = ask(host.planhost_splits, chunk(rng, D=D, bf16_rows=True), 4)
             assert (n, lo, size) == (1, 0, 0)
+
+
+def test_dequantize_once_takes_the_visible_keys_alone(host):
+    rng = random.Random(4)
+    seen_once = 0
+    for _ in range(4000):
+        c = chunk(rng)
+        if not c["library_scratch"]:
+            c["ws_bytes"] = rng.choice((0, 1 << 20, 1 << 33))
+        o = once(host, c)
+        a, b = seen(c)
+        if a > b:
+            assert not o["on"], c
+            continue
+        assert o["lo"] == a // 64 * 64 and o["lo"] + o["keys"] == b + 1, (c, o)
+        if not o["on"]:
+            continue
+        seen_once += 1
+        assert o["slab_rows"] == (-(-o["keys"] // 64) * 64 if o["tiled"] else o["keys"])
+        assert o["bytes"] == 4 * c["B"] * c["Hkv"] * o["slab_rows"] * c["D"]
+        assert c["library_scratch"] or o["bytes"] <= c["ws_bytes"]
+        assert o["tiled"] == (c["D"] >= 128) or not c["library_scratch"]
+    assert seen_once > 500
+
+
+@pytest.mark.parametrize("D", [256, 512])
+def test_a_window_over_a_long_cache_is_priced_by_its_own_keys(host, D):
+    # A few row blocks that see 1,000 of 60,000 keys.
+    c = dict(B=1, H=16, Hkv=8, L=300, D=D, total=60000, q_start=59700, k_start=0, causal=True,
+             window=700, blocks=-(-600 // ROWS[D]), bf16_rows=False, library_scratch=True,
+             ws_bytes=0)
+    o = once(host, c)
+    assert o["on"] == (D == 512)  # at D = 256 the rule for few blocks asks for 2,048 keys
+    assert o["keys"] < 1064 and o["lo"] + o["keys"] == 60000
+    if o["on"]:
+        assert o["bytes"] < 4 * 8 * 1100 * D
+
+
+def test_dequantize_once_never_takes_bf16_rows(host):
+    rng = random.Random(5)
+    for force in (-1, 1):
+        for _ in range(500):
+            assert not once(host, chunk(rng, bf16_rows=True), force)["on"]
