@@ -466,6 +466,8 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   const prefillplan::Once rows =
       prefillplan::dequantize_once(chunk, once_env ? strcmp(once_env, "0") != 0 : -1);
   bool once = rows.on;
+  if (once && slabs > prefillplan::kOnceMaxSlabs)
+    return fail(TQKV_EINVAL_SHAPE, "B * H_kv = %lld slabs", (long long)slabs);
   // Scratch that the call could do without (the partials; the rows of few
   // blocks) is left out where the library's cannot grow.
   void* ws = workspace;
@@ -484,7 +486,6 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   if (once) {
     uint16_t* kd = static_cast<uint16_t*>(ws);
     uint16_t* vd = kd + size_t(slabs) * size_t(rows.slab_rows) * size_t(D);
-    if (slabs > 65535) return fail(TQKV_EINVAL_SHAPE, "B * H_kv = %lld slabs", (long long)slabs);
     const Args d = keys_from(a, D, bits_k, bits_v, rows.lo, rows.keys);
     switch (D) {
       case 64: dequantize_rows<64>(d, bits_k, bits_v, slabs, rows.tiled, st, kd, vd); break;

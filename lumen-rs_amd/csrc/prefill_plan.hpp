@@ -65,6 +65,9 @@ inline int64_t once_blocks(int64_t D, int64_t keys) {
 }
 // The scratch that path may take; more keys dequantize in every block instead.
 constexpr size_t kOnceMaxBytes = size_t(4) << 30;
+// Slabs its launch takes. With more, fewer than kOnceBlocks row blocks stay in
+// block; a call of more blocks is refused.
+constexpr int64_t kOnceMaxSlabs = 65535;
 
 // Dequantize once: keys [lo, lo + keys) as slabs of slab_rows rows, V as
 // transposed tiles where `tiled`.
@@ -91,7 +94,8 @@ inline Once dequantize_once(const Chunk& c, int force) {
   o.slab_rows = once_slab_rows(o.tiled, o.keys);
   o.bytes = once_bytes(slabs, o.slab_rows, c.D);
   if (!c.library_scratch && c.ws_bytes < o.bytes) return o;
-  o.on = force == 1 || (c.blocks >= once_blocks(c.D, o.keys) &&
+  const int64_t few = slabs <= kOnceMaxSlabs ? once_blocks(c.D, o.keys) : kOnceBlocks;
+  o.on = force == 1 || (c.blocks >= few &&
                         once_bytes(slabs, o.keys, c.D) <= kOnceMaxBytes);
   return o;
 }

@@ -425,3 +425,19 @@ def test_prefill_window_over_a_long_cache_holds_little_scratch(T, monkeypatch, D
     want = want_mlx(q, cut(kh), cut(vh), 64, 4, 4, D ** -0.5, causal=True, q_start=1088 - L,
                     first_held=0, window=window)
     check(got, want, "window")
+
+
+def test_prefill_of_more_slabs_than_the_dequantize_pass_takes(T, monkeypatch):
+    # 65,536 (batch row, KV head) slabs at D = 512: one row block each, in block.
+    monkeypatch.delenv("TQKV_PREFILL_DEQUANT_ONCE", raising=False)
+    B, Hkv, L, N, D = 8192, 8, 1, 3, 512
+    q = kv_bf16((B, Hkv, L, D), 1)
+    k, v = (kv_bf16((B, Hkv, N, D), i) for i in (2, 3))
+    (kh, kd), (vh, vd) = _cache(k, 128, 4), _cache(v, 128, 4)
+    got = run(T, q, [(kd, vd, N, N, False)], B, Hkv, Hkv, L, D, 128, 4, 4, D ** -0.5, N - 1, 0,
+              True, -1)
+    for rows in (slice(0, 20), slice(B - 20, B)):
+        cut = lambda t: tuple(np.ascontiguousarray(a[rows]) for a in t)
+        want = want_mlx(np.ascontiguousarray(q[rows]), cut(kh), cut(vh), 128, 4, 4, D ** -0.5,
+                        causal=True, q_start=N - 1, first_held=0)
+        check(got[rows], want, f"slabs {rows.start}")

@@ -149,3 +149,12 @@ def test_dequantize_once_never_takes_bf16_rows(host):
     for force in (-1, 1):
         for _ in range(500):
             assert not once(host, chunk(rng, bf16_rows=True), force)["on"]
+
+
+def test_more_slabs_than_the_pass_takes_stay_in_block(host):
+    # Fewer than 8 row blocks over more than 65,535 slabs are attended in
+    # block; 8 or more are the pass's, whose launch refuses them.
+    c = dict(B=8192, H=8, Hkv=8, L=1, D=512, total=3, q_start=2, k_start=0, causal=True, window=-1,
+             blocks=1, bf16_rows=False, library_scratch=True, ws_bytes=0)
+    assert not once(host, c)["on"] and once(host, dict(c, B=8191))["on"]
+    assert not once(host, dict(c, blocks=7))["on"] and once(host, dict(c, blocks=8))["on"]
