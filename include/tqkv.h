@@ -185,8 +185,10 @@ typedef struct tqkv_affine_seg {
  * n_segs in {1, 2}.
  * workspace: device scratch of tqkv_decode_workspace_size() bytes for the
  * split partials, or NULL to use a buffer the library keeps per device (grown
- * on demand); calls that share a workspace must not overlap in time. One
- * kernel launch when B * H_kv fills the GPU, else a split launch plus a merge.
+ * on demand); calls that share a workspace must not overlap in time. At D =
+ * 512 with 4- or 8-bit K and V a smaller workspace (or library scratch that
+ * cannot grow, under a stream capture) may mean fewer splits, whose sums round
+ * differently. One kernel launch when B * H_kv fills the GPU, else a split launch plus a merge.
  * Returns TQKV_EUNSUPPORTED for a layout outside these sets.
  */
 int32_t tqkv_decode_attend_affine(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv,
@@ -200,7 +202,8 @@ int32_t tqkv_decode_attend_affine(const uint16_t* q, int32_t B, int32_t H, int32
  * reference. For callers that cannot call hipMalloc (code under HIP graph
  * capture, tight serving loops, harnesses that forbid it). Same arguments
  * and results (bit-identical: the same kernels and split plan) as
- * tqkv_decode_attend_affine without a workspace: the split partials live in
+ * tqkv_decode_attend_affine with a workspace of tqkv_decode_workspace_size()
+ * bytes, or without one where the library's scratch can grow: the split partials live in
  * a static device array of TQKV_NOALLOC_SCRATCH_BYTES that every device
  * running the library holds until the process ends. The first call on a
  * device looks up that device's copy (make it outside any graph capture);
@@ -378,7 +381,8 @@ int32_t tqkv_decode_attend_codebook_qjl(const uint16_t* q, int32_t B, int32_t H,
  * same bits. A chunk with too few row blocks to fill the GPU over more than
  * 1,024 keys that it can see splits the keys over workgroups, their partials
  * in the same scratch, and merges them (f32, so apart from the unsplit sums
- * by their rounding only). The mask is build_causal_mask_abs (native_attention.rs:
+ * by their rounding only); where the scratch cannot grow (under a stream
+ * capture) it does not split. The mask is build_causal_mask_abs (native_attention.rs:
  * 545-622) in absolute positions: query row l sits at q_start + l and key k
  * (counted across both segments) at k_start + k; with causal != 0, key k is
  * visible iff k_abs <= q_abs and, when window > 0, q_abs < k_abs + window

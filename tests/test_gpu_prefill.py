@@ -441,3 +441,40 @@ def test_prefill_of_more_slabs_than_the_dequantize_pass_takes(T, monkeypatch):
         want = want_mlx(np.ascontiguousarray(q[rows]), cut(kh), cut(vh), 128, 4, 4, D ** -0.5,
                         causal=True, q_start=N - 1, first_held=0)
         check(got[rows], want, f"slabs {rows.start}")
+
+
+@pytest.mark.parametrize("D,H,Hkv,L,P,S,window,bk,bv", [
+    (64, 8, 4, 20, 900, 1200, -1, 8, 4), (128, 16, 4, 33, 1300, 1500, -1, 4, 4),
+    (128, 8, 8, 10, 700, 2200, 1600, 3, 6), (256, 8, 2, 9, 1500, 700, -1, 4, 8),
+    (512, 32, 2, 7, 1111, 1500, -1, 4, 4), (512, 8, 4, 12, 600, 2600, 1900, 8, 4)])
+def test_prefill_key_splits_two_segments(T, monkeypatch, D, H, Hkv, L, P, S, window, bk, bv):
+    # A short chunk over a shared prefix and per-row suffixes, its keys split
+    # across the seam: the same bits dequantized once and in every block, the
+    # oracle's result, and, apart from the sums' rounding, what the entry that
+    # never splits gives.
+    B = 2
+    print(f"[prefill-splits] two segments D={D} L={L} P={P} S={S} window={window}", flush=True)
+    q = kv_bf16((B, H, L, D), S)
+    kp, vp = (kv_bf16((1, Hkv, P, D), S + i, frac=0.01, mult=10.0) for i in (1, 2))
+    ks, vs = (kv_bf16((B, Hkv, S, D), S + i, frac=0.01, mult=10.0) for i in (3, 4))
+    (kph, kpd), (vph, vpd) = _cache(kp, 64, bk), _cache(vp, 64, bv)
+    (ksh, ksd), (vsh, vsd) = _cache(ks, 64, bk, S + 3), _cache(vs, 64, bv, S + 3)
+    segs_host = [(kpd, vpd, P, P, True), (ksd, vsd, S + 3, S, False)]
+    args = (B, H, Hkv, L, D, 64, bk, bv, D ** -0.5)
+    got = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("TQKV_PREFILL_DEQUANT_ONCE", mode)
+        got[mode] = run(T, q, segs_host, *args, P + S - L, 0, True, window)
+    assert np.array_equal(got["0"], got["1"])
+    cat = lambda a, b: np.concatenate([np.broadcast_to(a, (B,) + a.shape[1:]), b], axis=2)
+    want = want_mlx(q, tuple(cat(a, b) for a, b in zip(kph, ksh)),
+                    tuple(cat(a, b) for a, b in zip(vph, vsh)), 64, bk, bv, D ** -0.5, causal=True,
+                    q_start=P + S - L, first_held=0, window=window)
+    check(got["1"], want, "splits, two segments")
+    dq = T.DeviceArray.of(q)
+    segs = [T.affine_seg(tuple(a.ptr for a in k), tuple(a.ptr for a in v), c, n, sh)
+            for (k, v, c, n, sh) in segs_host]
+    out = T.DeviceArray((B, H, L, D), np.uint16)
+    T.prefill_attend_affine_ws(dq.ptr, *args, segs, out.ptr, None, 0, P + S - L, 0, True, window)
+    T.hip().sync()
+    check(out.numpy(), want, "unsplit")

@@ -55,6 +55,25 @@ def test_noalloc_matches_workspace_entry(T, B, H, Hkv, D, bits, sizes):
         check_close(got, want)
 
 
+@pytest.mark.parametrize("B,H,Hkv,bits,N", [(1, 32, 2, 4, 3000), (2, 16, 4, 8, 700), (4, 32, 2, 4, 257),
+                                            (40, 16, 8, 4, 2000), (1, 32, 1, 4, 5000)])
+def test_wide_head_splits_do_not_depend_on_where_the_partials_go(T, B, H, Hkv, bits, N):
+    # Head dim 512 splits finer where there is room: the stated workspace, the
+    # library's scratch and the static array all have it, so the same bits.
+    D = 512
+    print(f"[noalloc] D=512 B={B} H={H}/{Hkv} bits={bits} N={N}", flush=True)
+    q = kv_bf16((B, H, 1, D), N)
+    (kh, kd), (vh, vd) = (_cache(kv_bf16((B, Hkv, N, D), N + i, frac=0.01, mult=10.0), 64, bits)
+                          for i in (1, 2))
+    ref, got = both(T, q, [(kd, vd, N, N, False)], B, H, Hkv, D, bits, bits, D ** -0.5, N)
+    out = T.DeviceArray((B, H, 1, D), np.uint16)
+    dq = T.DeviceArray.of(q)
+    seg = T.affine_seg(tuple(a.ptr for a in kd), tuple(a.ptr for a in vd), N, N)
+    T.decode_attend_affine(dq.ptr, B, H, Hkv, D, 64, bits, bits, D ** -0.5, [seg], out.ptr)
+    T.hip().sync()
+    assert np.array_equal(ref, got) and np.array_equal(ref, out.numpy())
+
+
 def test_noalloc_holds_no_library_scratch(T):
     """What the entry is for: on a shape that splits (config 1's layout, ~32
     splits a unit, so partials and a merge) it allocates nothing: with the
