@@ -232,9 +232,21 @@ void launch_encode(const uint16_t* x, int64_t s, int64_t rows, const float* R, i
                      dim3(unsigned((rows + 16 * MR - 1) / (16 * MR))), dim3(2 * D), 0, st, x, s, \
                      rows, R, mode, transpose, inner, bits, codes, sigma, dst_cap, dst_start, \
                      wide, words)
-  // 64 rows a workgroup read M a quarter as often; from 8,192 rows on they
-  // also fill the chip. At D = 64 (M is 16 KB) more wavefronts win.
-  if (D > 64 && rows > 8192)
+  // 64 rows a workgroup read M a quarter as often, but up to 16,384 rows (a
+  // workgroup a CU) they take the time of one workgroup: 17, 33 and 92 us at D =
+  // 128, 256 and 512, where 16 rows grow in rounds of 12,288, 8,192 and 4,096
+  // rows (what the CUs' LDS holds). R^T, 16 against 64 rows: D = 128, 16,384
+  // rows 18.1 and 17.1 us, 20,000 rows 20.3 and 21.7, 24,577 rows 23.3 and 21.9
+  // (R: 21.4 and 22.0, 32,768 rows 26.0 and 22.7); D = 256, 8,193 rows 32.5 and
+  // 33.2, 10,000 rows 35.2 and 33.7 (R, whose loads are coalesced as they are:
+  // 12,000 rows 31.3 and 33.7, 12,289 rows 36.4 and 34.2); D = 512, 8,192 rows
+  // 87 and 92, 8,193 rows 124 and 92. Mode 0 (no products): D = 256, 24,577 rows
+  // 19.9 and 22.6, 49,152 rows 36.4 and 35.1; D = 512, 12,289 rows 23.9 and
+  // 23.2. At D = 64 (M is 16 KB) more wavefronts win.
+  const int64_t most = D == 128 || (D == 256 && mode == 0) ? 24576
+                       : D == 256 && !transpose            ? 12288
+                                                           : 8192;
+  if (D > 64 && rows > most)
     TQKV_ENC(4);
   else
     TQKV_ENC(1);

@@ -293,10 +293,14 @@ def test_gpu_path_encode_bit_exact(T, mode, transpose, bits, D):
 @pytest.mark.parametrize("D,rows,mode,transpose,off", [
     (64, 17, 1, True, 0), (64, 8209, 1, False, 0), (128, 8192, 1, True, 0),
     (128, 8193, 1, True, 0), (128, 8255, 2, False, 2), (256, 8200, 1, False, 0),
-    (512, 8193, 2, True, 0), (512, 15, 1, True, 2), (256, 33, 0, False, 2)])
+    (512, 8193, 2, True, 0), (512, 15, 1, True, 2), (256, 33, 0, False, 2),
+    (128, 24576, 1, True, 0), (128, 24577, 1, True, 0), (128, 24600, 2, False, 2),
+    (256, 8193, 1, True, 2), (256, 12288, 2, False, 0), (256, 12289, 1, False, 0),
+    (256, 24583, 0, True, 0)])
 def test_gpu_path_encode_row_blocks(T, D, rows, mode, transpose, off):
-    # Both row-block sizes of the encode (16 rows, and 64 from 8,193 rows on
-    # at D > 64) and their remainders, on 16-byte aligned buffers and on ones
+    # Both row-block sizes of the encode (16 rows, and 64 at D = 128 from
+    # 24,577 rows on, at D = 256 from 8,193 with R^T, 12,289 with R and
+    # 24,577 without a rotation, at D = 512 from 8,193) and their remainders, on 16-byte aligned buffers and on ones
     # `off` bytes past that (element-wise loads and byte stores): codes and
     # sigma bit for bit, with a row of zeros (sigma 0, codes 0) and one whose
     # values are subnormal in bf16.
