@@ -438,7 +438,8 @@ int32_t prefill_launch(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, in
   const int64_t units = blocks * H_kv * B, q_rows = int64_t(B) * H * L;
   const size_t ws_bytes = workspace ? workspace_bytes : 0;
   const prefillplan::Chunk chunk{B, H, H_kv, L, D, a.total, q_start, k_start, a.causal != 0,
-                                 a.window, blocks, bf16_rows, library_scratch, ws_bytes};
+                                 a.window, rows_per_block, blocks, bf16_rows, library_scratch,
+                                 ws_bytes};
   size_t part_bytes = 0;
   const auto use_splits = [&](const prefillplan::Splits& sp) {
     a.n_splits = a.n_part = int(sp.n);

@@ -17,7 +17,8 @@ struct Chunk {
   int64_t q_start, k_start;
   bool causal;
   int64_t window;        // < 0: none
-  int64_t blocks;        // row blocks a KV head in the in-block kernel
+  int64_t block_rows;    // (position, head) rows a block of the in-block kernel
+  int64_t blocks;        // row blocks a KV head in it
   bool bf16_rows;        // K and V are bf16 rows, not packed codes
   bool library_scratch;  // else a caller's workspace, which holds rows only
   size_t ws_bytes;       // of that workspace
@@ -107,6 +108,11 @@ inline Once dequantize_once(const Chunk& c, int force) {
 // 24,000 keys 569 and 42 us, 147 rows over 16,384 565 and 55; D = 256, 256
 // rows over 16,384 661 and 104; 32 / 2 heads, D = 512, 64 rows over 20,000
 // 2,700 and 134 (with the wide kernel).
+// The keys a split holds are counted of what one row block sees: under a window
+// a block sees no more than the window and its own positions, and splits of
+// the chunk's whole range cost it their partials for nothing (D = 256, 8 heads,
+// 700 rows under a window of 512: 38 us unsplit, 47 in two splits of the range;
+// 300 rows under a window of 1,024: 44 us in two, 36 in three, even ones).
 // Not over bf16 rows: a codebook cache's dequantized rows and rotated queries
 // sit in the library scratch that the partials would take, and a bf16 cache's
 // chunk uses no scratch, so that caches on different streams stay independent.
@@ -127,15 +133,31 @@ inline Splits key_splits(const Chunk& c) {
   const int64_t units = c.blocks * c.H_kv * c.B, rows = c.B * c.H * c.L;
   if (c.bf16_rows || !c.library_scratch || units * 2 > kSplitWorkgroups) return s;
   const Visible v = visible_keys(c);
-  int64_t n = kSplitWorkgroups / units;
-  if (n > (v.hi - v.lo) / kSplitMinKeys) n = (v.hi - v.lo) / kSplitMinKeys;
+  const int64_t keys = v.hi + 1 - v.lo;
+  int64_t most = keys;  // that a row block sees
+  if (c.causal && c.window >= 0) {
+    const int64_t at = c.block_rows * c.H_kv / c.H + 1;  // positions it spans at most
+    const int64_t own = (at < c.L ? at : c.L) - 1;
+    if (most > c.window && most - c.window > own) most = c.window + own;
+  }
+  const int64_t room = kSplitWorkgroups / units;
+  int64_t n = room;
+  if (n > (most - 1) / kSplitMinKeys) n = (most - 1) / kSplitMinKeys;
+  if (n < 2) return s;
+  const auto whole = [](int64_t len) { return (len + kTileKeys - 1) / kTileKeys * kTileKeys; };
+  int64_t len = whole((most + n - 1) / n);
+  n = (keys + len - 1) / len;
+  if (most < keys) {  // the same number of splits, even over the whole range
+    if (n > room) n = room;
+    len = whole((keys + n - 1) / n);
+    n = (keys + len - 1) / len;
+  }
   const size_t slot = size_t(c.D + 2) * sizeof(float);
   if (n < 2 || size_t(rows) * size_t(n) * slot > kSplitMaxBytes) return s;
-  const int64_t keys = v.hi + 1 - v.lo;
-  s.len = (keys + n * kTileKeys - 1) / (n * kTileKeys) * kTileKeys;
-  s.n = (keys + s.len - 1) / s.len;
+  s.n = n;
+  s.len = len;
   s.lo = v.lo;
-  s.bytes = s.n > 1 ? size_t(rows) * size_t(s.n) * slot : 0;
+  s.bytes = size_t(rows) * size_t(n) * slot;
   return s;
 }
 

@@ -4,11 +4,11 @@
 
 using namespace tqkv::prefillplan;
 
-// c: B, H, H_kv, L, D, total, q_start, k_start, causal, window, blocks,
-// bf16_rows, library_scratch, ws_bytes.
+// c: B, H, H_kv, L, D, total, q_start, k_start, causal, window,
+// block_rows, blocks, bf16_rows, library_scratch, ws_bytes.
 static Chunk chunk(const int64_t* c) {
-  return Chunk{c[0], c[1], c[2], c[3], c[4],  c[5],       c[6],
-               c[7], c[8] != 0, c[9], c[10], c[11] != 0, c[12] != 0, size_t(c[13])};
+  return Chunk{c[0], c[1],      c[2], c[3],  c[4],  c[5],       c[6],       c[7],
+               c[8] != 0, c[9], c[10], c[11], c[12] != 0, c[13] != 0, size_t(c[14])};
 }
 
 extern "C" {

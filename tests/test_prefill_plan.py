@@ -10,8 +10,8 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BUILD = os.path.join(ROOT, "tests", "_build")
 LIB = os.path.join(BUILD, "libprefillplanhost.so")
-FIELDS = ("B", "H", "Hkv", "L", "D", "total", "q_start", "k_start", "causal", "window", "blocks",
-          "bf16_rows", "library_scratch", "ws_bytes")
+FIELDS = ("B", "H", "Hkv", "L", "D", "total", "q_start", "k_start", "causal", "window",
+          "block_rows", "blocks", "bf16_rows", "library_scratch", "ws_bytes")
 ROWS = {64: 128, 128: 256, 256: 128, 512: 64}  # rows a block of the in-block kernel
 
 
@@ -35,6 +35,12 @@ def once(host, c, force=-1):
                     ask(host.planhost_once, c, 6, force)))
 
 
+def blocked(c):
+    c["block_rows"] = ROWS[c["D"]]
+    c["blocks"] = -(-c["L"] * (c["H"] // c["Hkv"]) // ROWS[c["D"]])
+    return c
+
+
 def chunk(rng, **fixed):
     D = rng.choice((64, 128, 256, 512))
     Hkv = rng.choice((1, 2, 4, 8))
@@ -47,8 +53,7 @@ def chunk(rng, **fixed):
              library_scratch=rng.random() < 0.8, ws_bytes=0)
     c["q_start"] = rng.choice((c["k_start"] + total - L, 0, c["k_start"] + total // 2))
     c.update(fixed)
-    c["blocks"] = -(-c["L"] * (c["H"] // c["Hkv"]) // ROWS[c["D"]])
-    return c
+    return blocked(c)
 
 
 def seen(c):
@@ -135,9 +140,8 @@ def test_dequantize_once_takes_the_visible_keys_alone(host):
 def test_a_window_over_a_long_cache_is_priced_by_its_own_keys(host, D):
     # A few row blocks that see 1,000 of 60,000 keys.
     c = dict(B=1, H=16, Hkv=8, L=300, D=D, total=60000, q_start=59700, k_start=0, causal=True,
-             window=700, blocks=-(-600 // ROWS[D]), bf16_rows=False, library_scratch=True,
-             ws_bytes=0)
-    o = once(host, c)
+             window=700, bf16_rows=False, library_scratch=True, ws_bytes=0)
+    o = once(host, blocked(c))
     assert o["on"] == (D == 512)  # at D = 256 the rule for few blocks asks for 2,048 keys
     assert o["keys"] < 1064 and o["lo"] + o["keys"] == 60000
     if o["on"]:
@@ -155,6 +159,48 @@ def test_more_slabs_than_the_pass_takes_stay_in_block(host):
     # Fewer than 8 row blocks over more than 65,535 slabs are attended in
     # block; 8 or more are the pass's, whose launch refuses them.
     c = dict(B=8192, H=8, Hkv=8, L=1, D=512, total=3, q_start=2, k_start=0, causal=True, window=-1,
-             blocks=1, bf16_rows=False, library_scratch=True, ws_bytes=0)
+             block_rows=64, blocks=1, bf16_rows=False, library_scratch=True, ws_bytes=0)
     assert not once(host, c)["on"] and once(host, dict(c, B=8191))["on"]
     assert not once(host, dict(c, blocks=7))["on"] and once(host, dict(c, blocks=8))["on"]
+
+
+def test_a_window_splits_by_what_a_row_block_sees(host):
+    # A row block under a window sees the window and its own positions, however
+    # many keys the whole chunk sees: it takes two splits' keys or none is made.
+    base = dict(B=1, H=8, Hkv=8, L=700, D=256, total=1211, q_start=511, k_start=0, causal=True,
+                window=512, bf16_rows=False, library_scratch=True, ws_bytes=0)
+    assert ask(host.planhost_splits, blocked(dict(base)), 4)[0] == 1
+    assert ask(host.planhost_splits, blocked(dict(base, window=-1)), 4)[0] == 2
+    rng = random.Random(6)
+    split = 0
+    for _ in range(3000):
+        c = chunk(rng, causal=True, window=rng.choice((100, 600, 1024, 1500, 4000)))
+        n, ln = ask(host.planhost_splits, c, 4)[:2]
+        if n == 1:
+            continue
+        split += 1
+        sees = 0  # the most that a row block does
+        G, q0 = c["H"] // c["Hkv"], c["q_start"] - c["k_start"]
+        for r in range(0, c["L"] * G, c["block_rows"]):
+            first, last = r // G, (min(r + c["block_rows"], c["L"] * G) - 1) // G
+            a, b = max(0, q0 + first - c["window"] + 1), min(c["total"] - 1, q0 + last)
+            sees = max(sees, b - a + 1)
+        assert sees + 64 > 1024 and ln >= 256, (c, n, ln, sees)
+    assert split > 50
+
+
+def test_splits_without_a_window_are_even(host):
+    # At least 512 keys a split, at most 256 workgroups, whole tiles.
+    rng = random.Random(7)
+    for _ in range(3000):
+        c = chunk(rng, window=-1, library_scratch=True, k_start=0)
+        n, ln = ask(host.planhost_splits, c, 4)[:2]
+        a, b = seen(c)
+        keys, units = b + 1 - a, c["blocks"] * c["Hkv"] * c["B"]
+        want = min(256 // units, (keys - 1) // 512) if units <= 128 else 1
+        cut = -(-keys // (want * 64)) * 64 if want > 1 else 0
+        want = -(-keys // cut) if cut else 1
+        if want < 2 or c["B"] * c["H"] * c["L"] * want * (c["D"] + 2) * 4 > 1 << 30:
+            assert n == 1
+        else:
+            assert (n, ln) == (want, cut), c
