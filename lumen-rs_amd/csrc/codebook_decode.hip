@@ -26,8 +26,8 @@
 // more than the operands' last bits.
 // Measured a call: Gemma 4's global layers (B = 1, 32 / 2 heads, D = 512,
 // 32,768 tokens, 4-bit) 227 -> 43 us; B = 32, 16 / 8 heads, D = 256, 32,768
-// tokens, 3-bit 850 -> 803 us (5.4 TB/s; vector issue 68% of its cycles, LDS
-// 48%); B = 26, 8 heads, D = 128, 7,677 tokens 158 -> 109 us; B = 22, 32 / 8
+// tokens, 3-bit 850 -> 795 us (5.5 TB/s; vector issue 63% of its cycles, LDS
+// 43%); B = 26, 8 heads, D = 128, 7,677 tokens 158 -> 109 us; B = 22, 32 / 8
 // heads, D = 64, 31,445 tokens 293 -> 204 us. Wavefronts a SIMD (registers
 // against spills outside the loop): 4 at D = 256 (3: 860 us for the 3-bit
 // shape), 3 at D = 64 and 128 (4: 167 us for the D = 128 one), 2 at D = 512.
@@ -716,7 +716,8 @@ int32_t decode_codebook(const uint16_t* q, int32_t B, int32_t H, int32_t H_kv, i
                 (long long)cap);
   if (bits_k < 1 || bits_k > 8 || bits_v < 1 || bits_v > 8)
     return fail(TQKV_EUNSUPPORTED, "bits %d/%d", bits_k, bits_v);
-  // A lane loads D / 64 value codes at once (up to 4-byte words); key rows
+  // Value codes are copied 4 bytes at a time, at any alignment: what is asked
+  // of their pointer is the entry's stated contract, refused as ever. Key rows
   // are read 16 bytes a load (rows of D >= 64 bytes keep that alignment).
   const int v_align = D >= 256 ? 4 : D >= 128 ? 2 : 1;
   if (reinterpret_cast<uintptr_t>(v_codes) % v_align != 0)

@@ -4,17 +4,20 @@
 // (prefill_affine.hpp: the same products in the same order, the same 64-key
 // steps of the running maximum); this is its shape for wide heads.
 //
-// Bound: LDS reads. Each wavefront holds 16 query rows (Q, O and a tile's
-// scores then fit 256 registers at D = 512), so a K or V operand read (1 KB)
-// feeds one product: at 128 bytes a clock the reads of a tile take twice its
-// products' time, and at D = 512 the kernel runs at 98% of that read rate.
-// So nothing else may take LDS time or stall: the tiles go from HBM (mostly
-// L2: the blocks of a KV head share an XCD) straight into LDS, 16-byte
-// chunks permuted within their rows so that every operand read is free of
-// bank conflicts, with no staging registers; and no register spills (what
-// depends on the lane alone is recomputed a tile, see lane_now). The kernel
-// before it staged tiles through registers: at D = 512 that took one
-// wavefront a SIMD and 110 spilled registers.
+// Bound: no unit is full. Each wavefront holds 16 query rows (Q, O and a
+// tile's scores then fit 256 registers at D = 512), so a K or V operand read
+// (1 KB, 4 LDS cycles) feeds one product (16 cycles on one of four SIMDs): the
+// matrix cores and the LDS are each busy 60% of the kernel's cycles at D = 512
+// and 39% at D = 256 (counters), the vector units 30 and 34%. The rest is the
+// two wavefronts of a SIMD in the same phase (products, then softmax, then the
+// tile's barrier), and the clock, which the card holds at 1.84 GHz (D = 512)
+// and 2.07 (D = 256) of 2.4 under this load. So nothing else may stall:
+// the tiles go from HBM (mostly L2: the blocks of a KV head share an XCD)
+// straight into LDS, 16-byte chunks permuted within their rows so that every
+// operand read is free of bank conflicts (counter: 0), with no staging
+// registers; and no register spills (what depends on the lane alone is
+// recomputed a tile, see lane_now). The kernel before it staged tiles through
+// registers: at D = 512 that took one wavefront a SIMD and 110 spilled registers.
 // 32 rows a wavefront (half the LDS reads) measured 193 against 197 us at D
 // = 256 (sliding chunk, 2 x 32 heads, 3,071 keys) and needs twice the chunk
 // to fill the chip; at D = 512 it spills.
