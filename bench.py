@@ -1110,7 +1110,7 @@ def codebook_main(T, hip, args):
     alg = 2 * slabs * N * (D + 4) + 2 * B * H * D * 2 + D * D * 4
     result = _line(
         "codebook-cache decode tokens/s @ B=32, 32K ctx", B / (ms * 1e-3), "tokens/s", ms, args,
-        "bf16 in/out, f32 arithmetic",
+        "bf16 in/out, f16 hi + lo operands, f32 accumulate",
         {"workload": "config 2's shape (B=32, 16/8 heads, D=256, 32K context) over a TurboQuant "
                      "codebook cache: 3-bit Lloyd-Max codes (u8) + f32 sigma, K and V rotated",
          "batch": B, "q_heads": H, "kv_heads": HKV, "head_dim": D, "context": N,

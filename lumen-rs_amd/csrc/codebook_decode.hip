@@ -20,7 +20,7 @@
 // 4-byte LDS read: hi | lo << 16), where f32 multiply-adds a head repeated
 // the lookups for every two heads at D = 512 and cost a vector operation a
 // code and head. Against 64 bits the merged rows (before the rotation back and
-// the bf16 rounding) are 0.36 to 0.77 times as far off as that kernel's over 27
+// the bf16 rounding) are 0.36 to 0.80 times as far off as that kernel's over 81
 // shapes of every head dim, width and head count (D = 512, 16 heads: 2.8e-6 ->
 // 1.2e-6; D = 64: 1.2e-6 -> 1.0e-6): the f32 chain over D channels had lost
 // more than the operands' last bits.
