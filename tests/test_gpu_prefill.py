@@ -247,7 +247,7 @@ def test_prefill_wide_heads_match_in_block(T, monkeypatch, B, H, Hkv, D, L, N, q
 
 
 @pytest.mark.parametrize("B,H,Hkv,D,L,N,q_start,k_start,causal,window", [
-    (1, 8, 4, 64, 33, 1025, 992, 0, True, -1),      # two splits, the last 513 keys
+    (1, 8, 4, 64, 33, 1025, 992, 0, True, -1),      # two splits, of 576 and 449 keys
     (2, 16, 4, 128, 20, 2600, 2580, 0, True, -1),   # five
     (1, 8, 8, 128, 5, 4096, 0, 0, False, -1),       # eight, unmasked
     (1, 8, 8, 128, 40, 3000, 2900, 0, True, 1500),  # over the window's keys, rows with blind splits
